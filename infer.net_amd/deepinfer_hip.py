@@ -195,11 +195,18 @@ def _dp(t) -> Optional[int]:
 def _stream(stream) -> Optional[int]:
     """The stream handle to pass: an explicit stream, else torch's current stream. Torch's
     default stream is the HIP null stream (handle 0): it goes as NULL, which selects the
-    context's blocking stream, ordered against the null stream in both directions."""
+    context's blocking stream, ordered against the null stream in both directions.
+
+    The raw handle of the current device's stream costs 0.2 us; building the Stream object of
+    torch.cuda.current_stream() for its handle costs 2.9 us, the larger part of a small
+    call's 7.3 us on the host (a 4096 x 2048 GEMV's kernel takes 4.4 us)."""
     if stream is not None:
         return stream if isinstance(stream, int) else stream.cuda_stream
     try:
         import torch
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is not None and torch.cuda.is_initialized():
+            return raw(torch._C._cuda_getDevice())
         return torch.cuda.current_stream().cuda_stream
     except Exception:  # pragma: no cover - torch without a device
         return None

@@ -112,3 +112,13 @@ def test_null_stream_fill_before_prefill_moe(device):
     finally:
         for q in qs:
             q.dispose()
+
+
+def test_current_stream_handle(device):
+    """The stream handle a call without an explicit stream passes is the current stream's, on
+    torch's default stream (handle 0) and on a side stream."""
+    assert dh._stream(None) == torch.cuda.current_stream().cuda_stream == 0
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert dh._stream(None) == side.cuda_stream != 0
+    assert dh._stream(side) == side.cuda_stream and dh._stream(5) == 5
