@@ -151,8 +151,54 @@ bool launch_build_groups(const uint32_t *ids, int tokens, int experts, int with_
 // One block per token (prefill_merge gpu_prefill.mm:140-150): gate = sigmoid(shared_route .
 // x[t]); y = gate*out[T*8+t] + sum_{slot 0..7} p*out[t*8+slot]; residual[t] += y (f32 or
 // bf16 storage); with norm_w, normed[t] = r * rsqrt(mean(r^2) + eps) * norm_w over the
-// stored r (each thread re-reads only the elements it wrote).
-template <int BITS>
+// stored r.
+//
+// Bound by latency for short chunks and by the route outputs (9*H*4 bytes a token) for long
+// ones. A thread owns VEC consecutive columns of each 256*VEC, two such pieces at a time: the
+// nine route rows, the residual and the norm weights of the first two pieces (all of a
+// 2048-wide row) are requested before the shared-expert gate's dot product, whose wait and
+// barrier they then cover, and a row of up to kMergeHold pieces keeps its stored r in
+// registers for the norm. VEC 4 needs every row 16-byte aligned (8-byte for bf16), VEC 1
+// takes any other caller buffers. Against one column a thread at a time behind the gate: a
+// 77-token 5-bit layer with norm 143.2 -> 138.6 us, 2048 tokens 349.9 -> 343.6 us, 512 tokens
+// without norm 243.5 -> 241.5 us.
+constexpr int kMergeHold = 2;
+
+// VEC consecutive elements of an f32 or bf16 row.
+template <int VEC>
+DIH_DEV void row_load(float (&v)[VEC], const void *p, int f32, size_t at) {
+    if constexpr (VEC == 4) {
+        if (f32) {
+            const dih_f32x4 q = *reinterpret_cast<const dih_f32x4 *>(static_cast<const float *>(p) + at);
+            v[0] = q[0]; v[1] = q[1]; v[2] = q[2]; v[3] = q[3];
+        } else {
+            const uint2 q = *reinterpret_cast<const uint2 *>(static_cast<const uint16_t *>(p) + at);
+            v[0] = __uint_as_float(q.x << 16); v[1] = __uint_as_float(q.x & 0xffff0000u);
+            v[2] = __uint_as_float(q.y << 16); v[3] = __uint_as_float(q.y & 0xffff0000u);
+        }
+    } else {
+        v[0] = residual_load(p, f32, at);
+    }
+}
+
+// Stores them; v becomes what was stored (rounded to bf16).
+template <int VEC>
+DIH_DEV void row_store(float (&v)[VEC], void *p, int f32, size_t at) {
+    if constexpr (VEC == 4) {
+        if (f32) {
+            *reinterpret_cast<dih_f32x4 *>(static_cast<float *>(p) + at) = dih_f32x4{v[0], v[1], v[2], v[3]};
+        } else {
+            const uint2 q = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+            *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(p) + at) = q;
+            v[0] = __uint_as_float(q.x << 16); v[1] = __uint_as_float(q.x & 0xffff0000u);
+            v[2] = __uint_as_float(q.y << 16); v[3] = __uint_as_float(q.y & 0xffff0000u);
+        }
+    } else {
+        v[0] = residual_store(p, f32, at, v[0]);
+    }
+}
+
+template <int BITS, int VEC>
 __global__ __launch_bounds__(256) void merge_kernel(const uint32_t *sr_packed,
                                                     const uint16_t *sr_scales,
                                                     const uint16_t *sr_biases,
@@ -163,95 +209,171 @@ __global__ __launch_bounds__(256) void merge_kernel(const uint32_t *sr_packed,
     __shared__ float sq[4];
     const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nchunk = H >> 5;
+    const int np = H / VEC;   // pieces of a row (H is a multiple of 64)
+    const float *sh = route_out + ((size_t)tokens * 8 + t) * H;
+    const float *ro = route_out + (size_t)t * 8 * H;
+    const size_t row = (size_t)t * H;
+    // this thread's pieces p0 and p0 + 256 (clamped in bounds; pieces past the row are not
+    // stored): shared row, eight route rows, residual
+    float in[2][9][VEC], res[2][VEC], nw[2][VEC];
+    auto load = [&](int p0) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int c = VEC * min(p0 + 256 * k, np - 1);
+            row_load<VEC>(in[k][8], sh, 1, c);
+#pragma unroll
+            for (int s = 0; s < 8; s++) row_load<VEC>(in[k][s], ro + (size_t)s * H, 1, c);
+            row_load<VEC>(res[k], residual, mo.residual_f32, row + c);
+        }
+    };
+    float p[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++) p[s] = probs[(size_t)t * 8 + s];
+    // the gate's operands first: its wait then leaves the rows in flight
+    Chunk<BITS> c0;
+    float xr[32];
+    uint32_t sc0 = 0, bi0 = 0;
+    if (tid < nchunk) {
+        load_chunk<BITS>(c0, sr_packed, tid);
+        sc0 = sr_scales[tid >> 1];
+        bi0 = sr_biases[tid >> 1];
+        load_x32(xr, x + row, 1, tid * 32);
+    }
+    load(tid);
+    if (mo.norm_w) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) row_load<VEC>(nw[k], mo.norm_w, 1, VEC * min(tid + 256 * k, np - 1));
+    }
+    // (a row has at most 256 chunks: one a thread)
     float d = 0.f;
-    for (int ch = tid; ch < nchunk; ch += 256) {
-        Chunk<BITS> c;
-        load_chunk<BITS>(c, sr_packed, ch);
-        float xr[32];
-        load_x32(xr, x + (size_t)t * H, 1, ch * 32);
+    if (tid < nchunk) {
         float xs = 0.f;
 #pragma unroll
         for (int i = 0; i < 32; i++) xs += xr[i];
-        d += bf16_to_f32(sr_scales[ch >> 1]) * chunk_dot<BITS>(c, xr) + bf16_to_f32(sr_biases[ch >> 1]) * xs;
+        d = bf16_to_f32(sc0) * chunk_dot<BITS>(c0, xr) + bf16_to_f32(bi0) * xs;
     }
     d = wave_sum(d);
     if (lane == 0) part[wave] = d;
     __syncthreads();
     const float gate = sigmoidf_((part[0] + part[1]) + (part[2] + part[3]));
-    float p[8];
-#pragma unroll
-    for (int s = 0; s < 8; s++) p[s] = probs[(size_t)t * 8 + s];
     // a token whose router logits were not finite (NaN probabilities) keeps its residual
     // and normed row unchanged (uniform over the block: one token)
     if (__builtin_isnan(p[0])) return;
-    const float *sh = route_out + ((size_t)tokens * 8 + t) * H;
-    const float *ro = route_out + (size_t)t * 8 * H;
     float ss = 0.f;
-    for (int c = tid; c < H; c += 256) {
-        float y = sh[c] * gate;
+    for (int p0 = tid; p0 < np; p0 += 512) {
+        if (p0 != tid) load(p0);
 #pragma unroll
-        for (int s = 0; s < 8; s++) y += ro[(size_t)s * H + c] * p[s];
-        const size_t at = (size_t)t * H + c;
-        const float r = residual_store(residual, mo.residual_f32, at, residual_load(residual, mo.residual_f32, at) + y);
-        ss += r * r;
+        for (int k = 0; k < 2; k++) {
+            if (p0 + 256 * k >= np) continue;
+#pragma unroll
+            for (int j = 0; j < VEC; j++) {
+                float y = in[k][8][j] * gate;
+#pragma unroll
+                for (int s = 0; s < 8; s++) y += in[k][s][j] * p[s];
+                res[k][j] += y;
+            }
+            row_store<VEC>(res[k], residual, mo.residual_f32, row + VEC * (p0 + 256 * k));
+#pragma unroll
+            for (int j = 0; j < VEC; j++) ss += res[k][j] * res[k][j];
+        }
     }
     if (!mo.norm_w) return;  // uniform over the launch
     ss = wave_sum(ss);
     if (lane == 0) sq[wave] = ss;
     __syncthreads();
     const float scale = rsqrtf(((sq[0] + sq[1]) + (sq[2] + sq[3])) / (float)H + mo.eps);
-    for (int c = tid; c < H; c += 256) {
-        const size_t at = (size_t)t * H + c;
-        const float v = residual_load(residual, mo.residual_f32, at) * scale * mo.norm_w[c];
-        if (mo.normed_f32) static_cast<float *>(mo.normed)[at] = v;
-        else static_cast<uint16_t *>(mo.normed)[at] = f32_to_bf16(v);
+    const bool held = np <= 256 * kMergeHold;
+    for (int p0 = tid; p0 < np; p0 += 512) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int pc = p0 + 256 * k;
+            if (pc >= np) continue;
+            if (!held) {   // (each thread re-reads only the elements it wrote)
+                row_load<VEC>(res[k], residual, mo.residual_f32, row + VEC * pc);
+                row_load<VEC>(nw[k], mo.norm_w, 1, VEC * pc);
+            }
+            float v[VEC];
+#pragma unroll
+            for (int j = 0; j < VEC; j++) v[j] = res[k][j] * scale * nw[k][j];
+            row_store<VEC>(v, mo.normed, mo.normed_f32, row + VEC * pc);
+        }
     }
+}
+
+// Whether rows of `H` elements (a multiple of 64) from p can be read four elements at a time.
+static bool rows_by_four(const void *p, int f32) {
+    return (reinterpret_cast<uintptr_t>(p) & (f32 ? 15 : 7)) == 0;
 }
 
 bool launch_moe_merge(const Matrix *shared_route, const uint16_t *x, int tokens, int hidden,
                       const float *route_out, const float *probs, void *residual,
                       const MergeOut &mo, hipStream_t s, char *error, int capacity) {
-    if (shared_route->bits == 8)
-        DIH_LAUNCH((merge_kernel<8>), dim3(tokens), dim3(256), 0, s, shared_route->packed(),
-                           shared_route->scales(), shared_route->biases(), x, tokens, hidden, route_out,
-                           probs, residual, mo);
-    else
-        DIH_LAUNCH((merge_kernel<5>), dim3(tokens), dim3(256), 0, s, shared_route->packed(),
-                           shared_route->scales(), shared_route->biases(), x, tokens, hidden, route_out,
-                           probs, residual, mo);
+    const bool four = rows_by_four(route_out, 1) && rows_by_four(residual, mo.residual_f32) &&
+                      (!mo.norm_w || (rows_by_four(mo.norm_w, 1) && rows_by_four(mo.normed, mo.normed_f32)));
+#define DIH_MERGE_CASE(B, V)                                                                                  \
+    if (shared_route->bits == B && four == (V == 4))                                                          \
+        DIH_LAUNCH((merge_kernel<B, V>), dim3(tokens), dim3(256), 0, s, shared_route->packed(),               \
+                   shared_route->scales(), shared_route->biases(), x, tokens, hidden, route_out, probs,       \
+                   residual, mo);
+    DIH_MERGE_CASE(8, 4) DIH_MERGE_CASE(8, 1) DIH_MERGE_CASE(5, 4) DIH_MERGE_CASE(5, 1)
+#undef DIH_MERGE_CASE
     return hip_ok(hipGetLastError(), error, capacity, "merge launch");
 }
 
 // ---------------------------------------------------------------------------- norm
 
 // One block per token: normed[t] = r[t] * rsqrt(sum(r[t]^2)/H + eps) * w (the norm of
-// graph_merge_norm / prefill_add_norm, gpu_graph.mm:40-61).
-__global__ __launch_bounds__(256) void rmsnorm_kernel(const void *r, int r_f32, int H, const float *w,
-                                                      float eps, void *out, int out_f32, const float *probs) {
-    __shared__ float sq[4];
+// graph_merge_norm / prefill_add_norm, gpu_graph.mm:40-61). Bound by latency (one block for
+// the decode token): each of 1024 threads requests its N residual and N weight elements at
+// once, one memory round trip, and keeps them (N = 2 up to 2048 columns, 8 up to 8192). The
+// decode step with norm went 19.7 -> 17.1 us (8-bit) and 19.0 -> 16.7 us (5-bit) against 256
+// threads reading eight elements each, twice.
+template <int N>
+__global__ __launch_bounds__(1024) void rmsnorm_kernel(const void *r, int r_f32, int H, const float *w,
+                                                       float eps, void *out, int out_f32, const float *probs) {
+    __shared__ float sq[16];
     const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // the token's merge was skipped (non-finite router logits): its normed row stays as it was
-    if (probs && __builtin_isnan(probs[(size_t)t * 8])) return;
-    float ss = 0.f;
-    for (int c = tid; c < H; c += 256) {
-        const float v = residual_load(r, r_f32, (size_t)t * H + c);
-        ss += v * v;
+    const float p0 = probs ? probs[(size_t)t * 8] : 0.f;
+    float v[N], wv[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const int c = min(tid + 1024 * k, H - 1);
+        v[k] = residual_load(r, r_f32, (size_t)t * H + c);
+        wv[k] = w[c];
     }
+    // the token's merge was skipped (non-finite router logits): its normed row stays as it was
+    if (__builtin_isnan(p0)) return;
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < N; k++) ss += tid + 1024 * k < H ? v[k] * v[k] : 0.f;
     ss = wave_sum(ss);
     if (lane == 0) sq[wave] = ss;
     __syncthreads();
-    const float scale = rsqrtf(((sq[0] + sq[1]) + (sq[2] + sq[3])) / (float)H + eps);
-    for (int c = tid; c < H; c += 256) {
+    float total = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; k++) total += sq[k];
+    const float scale = rsqrtf(total / (float)H + eps);
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const int c = tid + 1024 * k;
+        if (c >= H) continue;
         const size_t at = (size_t)t * H + c;
-        const float v = residual_load(r, r_f32, at) * scale * w[c];
-        if (out_f32) static_cast<float *>(out)[at] = v;
-        else static_cast<uint16_t *>(out)[at] = f32_to_bf16(v);
+        const float o = v[k] * scale * wv[k];
+        if (out_f32) static_cast<float *>(out)[at] = o;
+        else static_cast<uint16_t *>(out)[at] = f32_to_bf16(o);
     }
 }
 
 bool launch_rmsnorm(const void *r, int r_f32, int tokens, int hidden, const float *w, float eps,
                     void *out, int out_f32, const float *probs, hipStream_t s, char *error, int capacity) {
-    DIH_LAUNCH(rmsnorm_kernel, dim3(tokens), dim3(256), 0, s, r, r_f32, hidden, w, eps, out, out_f32, probs);
+    if (hidden <= 2048)
+        DIH_LAUNCH((rmsnorm_kernel<2>), dim3(tokens), dim3(1024), 0, s, r, r_f32, hidden, w, eps, out, out_f32, probs);
+    else if (hidden <= 8192)
+        DIH_LAUNCH((rmsnorm_kernel<8>), dim3(tokens), dim3(1024), 0, s, r, r_f32, hidden, w, eps, out, out_f32, probs);
+    else {
+        set_error(error, capacity, "Norm rows wider than 8192 are not supported");
+        return false;
+    }
     return hip_ok(hipGetLastError(), error, capacity, "norm launch");
 }
 

@@ -43,7 +43,8 @@ def _check(res, normed, r0, y, w, eps, res_f32, normed_f32):
 
 @pytest.mark.parametrize("res_f32,normed_f32", [(True, True), (False, False), (True, False)])
 @pytest.mark.parametrize("bits,E,H,I", [(8, 256, 2048, 512), (5, 256, 2048, 512),
-                                        (8, 16, 1024, 1536)])   # I > 1024: the GEMV-stage path
+                                        (8, 16, 1024, 1536),    # I > 1024: the GEMV-stage path
+                                        (8, 8, 4096, 64)])      # a row past 2048 columns
 def test_decode_merge_norm(device, bits, E, H, I, res_f32, normed_f32):
     rng = np.random.default_rng(40 + bits + I)
     L = _moe_layer(rng, E, H, I, bits)
@@ -221,6 +222,65 @@ def test_prefill_nonfinite_logit_leaves_its_token_unchanged(device, bits, T):
         assert np.array_equal(res[~good], r0[~good]) and (normed[~good] == 3.0).all()
         assert np.array_equal(ids[good], clean[2][good])
         assert np.array_equal(res[good], clean[0][good]) and np.array_equal(normed[good], clean[1][good])
+    finally:
+        for m in q:
+            if m is not None:
+                m.dispose()
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("res_f32", [True, False])
+@pytest.mark.parametrize("H", [64, 1088, 2048, 2112, 4096])
+def test_prefill_merge_widths_and_alignment(device, H, res_f32, offset):
+    """The merge and its norm over row widths around a block's pieces (one piece, a ragged
+    second piece, rows that are re-read for the norm), with buffers on 16-byte boundaries and
+    one element off them, against the f64 merge of the route outputs the call itself reports:
+    nine f32 products and sums a column, at most 16 roundings of 2^-24 of the terms' sum."""
+    rng = np.random.default_rng(H + offset)
+    T, E, I, eps = 5, 8, 64, 1e-6
+    L = _moe_layer(rng, E, H, I, 8, router=False)
+    q, layer = _upload_layer(device, L)
+
+    def shifted(values, dtype):
+        flat = torch.zeros(values.size + 8, dtype=dtype, device="cuda")
+        view = flat[offset:offset + values.size].view(values.shape)
+        view.copy_(torch.from_numpy(np.ascontiguousarray(values)))
+        return view
+
+    try:
+        xb = orc.f32_to_bf16_bits(rng.normal(size=(T, H)).astype(np.float32))
+        lb = orc.f32_to_bf16_bits(rng.normal(size=(T, E)).astype(np.float32))
+        r0 = rng.normal(size=(T, H)).astype(np.float32)
+        if not res_f32:
+            r0 = orc.bf16_bits_to_f32(orc.f32_to_bf16_bits(r0))
+        w = rng.uniform(0.5, 1.5, size=H).astype(np.float32)
+        dtype = torch.float32 if res_f32 else torch.bfloat16
+        res, normed = shifted(r0, dtype), shifted(np.zeros((T, H), np.float32), dtype)
+        weight = shifted(w, torch.float32)
+        rout = torch.zeros((T * 9, H), dtype=torch.float32, device="cuda")
+        probs = torch.zeros((T, 8), dtype=torch.float32, device="cuda")
+        dh.moe_prefill(device, layer, T, dev_bf16(xb), dev_bf16(lb), res,
+                       trace=dh.make_trace(expert_out=rout, probs=probs),
+                       merge=dh.make_merge(res_f32, weight, eps, normed, res_f32))
+        torch.cuda.synchronize()
+        xf = orc.bf16_bits_to_f32(xb).astype(np.float64)
+        gate = 1.0 / (1.0 + np.exp(-orc.dense_f64(L.shared_route, xf.astype(np.float32), round_operands=False)))
+        ro = rout.cpu().numpy().astype(np.float64)
+        terms = np.concatenate([ro[:T * 8].reshape(T, 8, H) * probs.cpu().numpy()[:, :, None],
+                                (ro[T * 8:] * gate)[:, None, :]], axis=1)
+        want = r0 + terms.sum(axis=1)
+        got = res.float().cpu().numpy().astype(np.float64)
+        # (the gate is an f32 dot product and exponential: 1e-5 of the shared row)
+        bound = 16 * 2.0 ** -24 * (np.abs(terms).sum(axis=1) + np.abs(r0)) + 1e-5 * np.abs(terms[:, 8])
+        if not res_f32:
+            bound += 2.0 ** -8 * np.abs(want)
+        assert (np.abs(got - want) <= bound).all(), np.max(np.abs(got - want) - bound)
+        _, want_n = orc.merge_norm_f64(got, np.zeros_like(got), w, eps)
+        got_n = normed.float().cpu().numpy()
+        if res_f32:
+            assert orc.rel_err(got_n, want_n) < 1e-5
+        else:
+            assert_rounded(got_n, want_n, 0.0)
     finally:
         for m in q:
             if m is not None:
