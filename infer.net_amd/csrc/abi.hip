@@ -151,6 +151,20 @@ static hipStream_t pick(Context *c, void *stream) {
     return stream ? static_cast<hipStream_t>(stream) : c->stream;
 }
 
+// Split-K planes for a dense call on `s`, or null: a stream past the slots, or one under
+// capture (a graph's kernels would keep the slot of the capturing stream and could replay
+// beside that stream's own calls).
+static float *dense_planes(Context *c, hipStream_t s) {
+    if (!c->planes) return nullptr;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return nullptr;
+    int i = 0;
+    while (i < c->plane_used && c->plane_stream[i] != s) i++;
+    if (i == Context::kPlaneSlots) return nullptr;
+    if (i == c->plane_used) c->plane_stream[c->plane_used++] = s;
+    return reinterpret_cast<float *>(c->planes + (size_t)i * Context::kPlaneBytes);
+}
+
 static bool stage(Matrix *m, size_t in_floats, size_t out_floats, char *error, int capacity) {
     if (m->stage_in_bytes < in_floats * 4) {
         if (m->stage_in) (void)hipFree(m->stage_in);
@@ -231,6 +245,11 @@ __attribute__((visibility("default"))) void *dih_quant_create_configured(int res
         delete c;
         return nullptr;
     }
+    // (without the planes dense calls run unsplit)
+    if (hipMalloc(reinterpret_cast<void **>(&c->planes), Context::kPlaneSlots * Context::kPlaneBytes) != hipSuccess) {
+        c->planes = nullptr;
+        (void)hipGetLastError();
+    }
     return c;
 }
 
@@ -244,6 +263,7 @@ __attribute__((visibility("default"))) void dih_quant_destroy(void *p) {
     (void)hipStreamSynchronize(c->stream);
     for (auto &s : c->ws)
         if (s.ptr) (void)hipFree(s.ptr);
+    if (c->planes) (void)hipFree(c->planes);
     for (auto &e : c->prof_pool) (void)hipEventDestroy(e);
     (void)hipEventDestroy(c->start);
     (void)hipEventDestroy(c->stop);
@@ -1128,17 +1148,9 @@ __attribute__((visibility("default"))) int dih_dense(void *ctx, void *matrix, in
     ProfScope prof_scope(c);
     // Dispatch policy (p_gemv, gpu_prefill.mm:603-620, picks GEMV kernels below 64 tokens):
     // up to kDenseGemvTokens tokens run as one batched GEMV launch (each token a slot of
-    // expert 0; measured 8 / 13 / 18 us against 26 us for the MFMA tile at 1 / 2 / 4 tokens
-    // of an 8192 x 2048 8-bit matrix), long chunks as the bf16 GEMM after one dequantization
-    // pass (the fused tile re-dequantizes the weights for every 128 tokens), the rest as the
-    // fused MFMA GEMM.
+    // expert 0; it multiplies unrounded weights, so where it ends is also a rounding point),
+    // longer chunks on bf16 MFMAs as dense_plan chooses.
     constexpr int kDenseGemvTokens = 4;
-    if (tokens >= 1024 || (tokens >= 512 && m->rows <= 4096)) {
-        bool ok = launch_dense_gemm(c, m, tokens, static_cast<const uint16_t *>(x), y, y_dtype == DIH_BF16, s,
-                                    error, capacity);
-        prof_mark(c, s, "dense_qmm");
-        return ok ? 0 : -1;
-    }
     if (tokens <= kDenseGemvTokens) {
         QmvSeg sg = seg_of(m);
         sg.count = tokens; sg.x = x; sg.x_bf16 = 1; sg.x_slot_stride = m->columns;
@@ -1148,6 +1160,15 @@ __attribute__((visibility("default"))) int dih_dense(void *ctx, void *matrix, in
         return ok ? 0 : -1;
     }
     QmmArgs a;
+    a.part = dense_planes(c, s);
+    a.part_bytes = a.part ? Context::kPlaneBytes : 0;
+    a.plan = dense_plan(m, tokens, a.part_bytes);
+    if (a.plan.gemm) {
+        bool ok = launch_dense_gemm(c, m, tokens, static_cast<const uint16_t *>(x), y, y_dtype == DIH_BF16, s,
+                                    error, capacity);
+        prof_mark(c, s, "dense_qmm");
+        return ok ? 0 : -1;
+    }
     a.m0 = m; a.tokens = tokens; a.dense = 1; a.x = static_cast<const uint16_t *>(x); a.in_mode = 0;
     a.y = y; a.y_bf16 = y_dtype == DIH_BF16;
     bool ok = launch_qmm(a, s, error, capacity);

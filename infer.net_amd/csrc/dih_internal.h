@@ -70,6 +70,14 @@ struct Context {
     int prof_used = 0;                        // events taken from the pool since reset
     // named scratch
     Scratch ws[32];
+    // Split-K planes of dih_dense, one slot per stream (the first kPlaneSlots streams that
+    // ask; others run unsplit), so that dense calls on different streams of one context stay
+    // independent of each other. Allocated with the context, freed with it.
+    static constexpr int kPlaneSlots = 4;
+    static constexpr size_t kPlaneBytes = (size_t)32 << 20;
+    char *planes = nullptr;
+    hipStream_t plane_stream[kPlaneSlots] = {};
+    int plane_used = 0;
     // this device's copy of the fixed scratch array of dih_moe_decode_noalloc (its device
     // address, looked up once per device), or null with the lookup's error
     void *noalloc = nullptr;
@@ -174,6 +182,16 @@ bool launch_top8(const void *logits, int logits_bf16, int tokens, int experts, u
 bool launch_build_groups(const uint32_t *ids, int tokens, int experts, int with_shared,
                          uint32_t *counts, uint32_t *routes, hipStream_t s, char *error, int capacity);
 
+// How a dense projection of more than the GEMV's tokens runs: dequantize + bf16 GEMM, or the
+// fused streaming kernel with `nt` 32-token tiles a block and K in `ksplit` ranges (nt 0: the
+// general fused kernel).
+struct DensePlan {
+    bool gemm = false;
+    int nt = 0, ksplit = 1;
+};
+// The fastest by estimate; part_bytes: split-K planes available (0: no ranges).
+DensePlan dense_plan(const Matrix *m, int tokens, size_t part_bytes);
+
 struct QmmArgs {
     // routed matrices (gate or down) and optional up for the gated kernel
     const Matrix *m0 = nullptr, *m1 = nullptr;
@@ -187,6 +205,8 @@ struct QmmArgs {
     const uint16_t *x = nullptr;        // bf16 input rows
     int in_mode = 0;                    // 0: row = route; 1: gate input row (route/8, shared)
     void *y = nullptr; int y_bf16 = 0;  // output rows indexed by route
+    DensePlan plan;                     // dense: from dense_plan
+    float *part = nullptr; size_t part_bytes = 0;   // and its split-K planes (optional)
 };
 bool launch_qmm(const QmmArgs &a, hipStream_t s, char *error, int capacity);
 // The grouped gate/up launch of `tokens` tokens over `gate` takes the wide (96/128-route)
@@ -258,6 +278,7 @@ size_t attention_score_floats(int position, int tokens, int round, int partition
 // then the library's bf16 MFMA GEMM with f32 accumulation, Y[T][R] = X[T][C] * W16[R][C]^T.
 bool launch_dense_gemm(Context *c, const Matrix *m, int tokens, const uint16_t *x, void *y, bool y_bf16,
                        hipStream_t s, char *error, int capacity);
+void gemm_tile(int R, int T, int &bm, int &bn);   // its block shape: weight rows, tokens
 bool launch_gemm_bf16(const uint16_t *w16, int R, int C, int tokens, const uint16_t *x, void *y, bool y_bf16,
                       hipStream_t s, char *error, int capacity);
 bool launch_dequant_bf16_rows(const uint32_t *packed, const uint16_t *scales, const uint16_t *biases, int bits,

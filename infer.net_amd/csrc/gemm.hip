@@ -385,6 +385,19 @@ size_t tiles_of(int R, int T, int bm, int bn) { return (size_t)((R + bm - 1) / b
 
 }  // namespace
 
+// The largest block shape whose tiles still give about one per CU.
+void gemm_tile(int R, int T, int &bm, int &bn) {
+    constexpr size_t kFill = 240;
+    bm = 256;
+    bn = 256;
+    if (tiles_of(R, T, bm, bn) >= kFill) return;
+    bn = 128;
+    if (tiles_of(R, T, bm, bn) >= kFill) return;
+    bm = 128;
+    if (tiles_of(R, T, bm, bn) >= kFill) return;
+    bn = 64;
+}
+
 bool launch_dequant_bf16_rows(const uint32_t *packed, const uint16_t *scales, const uint16_t *biases, int bits,
                               int rows, int columns, uint16_t *out, hipStream_t s, char *error, int capacity) {
     const size_t items = (size_t)rows * (bits == 8 ? columns / 16 : columns / 32);
@@ -413,11 +426,11 @@ bool launch_gemm_bf16(const uint16_t *w16, int R, int C, int tokens, const uint1
     }
     GemmParams p{};
     p.w = w16; p.x = x; p.y = y; p.R = R; p.T = tokens; p.C = C; p.y_bf16 = y_bf16 ? 1 : 0;
-    // the largest block shape whose tiles still give about one per CU
-    constexpr size_t kFill = 240;
-    if (tiles_of(R, tokens, 256, 256) >= kFill) return run_gemm<4, 2, 2, 4, 2, 64>(p, 8, s, error, capacity);
-    if (tiles_of(R, tokens, 256, 128) >= kFill) return run_gemm<4, 2, 2, 2, 2, 64>(p, 8, s, error, capacity);
-    if (tiles_of(R, tokens, 128, 128) >= kFill) return run_gemm<2, 2, 2, 2, 4, 64>(p, 8, s, error, capacity);
+    int bm, bn;
+    gemm_tile(R, tokens, bm, bn);
+    if (bn == 256) return run_gemm<4, 2, 2, 4, 2, 64>(p, 8, s, error, capacity);
+    if (bm == 256) return run_gemm<4, 2, 2, 2, 2, 64>(p, 8, s, error, capacity);
+    if (bn == 128) return run_gemm<2, 2, 2, 2, 4, 64>(p, 8, s, error, capacity);
     return run_gemm<2, 2, 2, 1, 4, 64>(p, 8, s, error, capacity);
 }
 

@@ -53,6 +53,7 @@ struct QmmParams {
     const uint32_t *routes;            // [ngroups * tokens]
     const uint32_t *counts;            // [ngroups]
     int max_work;                      // grid work items (upper bound)
+    int ksplit, ksteps;                // split-K dense launches: K ranges, K steps of each
     const uint16_t *x; void *y;
 };
 
@@ -375,9 +376,6 @@ constexpr int qmm_lds_occupancy() {
 // SPLIT (gated only): eight waves, waves 0-3 the gate matrix and 4-7 the up matrix of the
 // same four 32-row slabs, so that two waves share each SIMD and one's dequant overlaps the
 // other's MFMAs and waits; the SwiGLU epilogue meets the two halves in LDS.
-// RS (dense only): 32-row slabs per wave, so a block's row tile is 128*RS rows. Two slabs
-// double the MFMA work per activation tile read from LDS (each wave reads the whole tile
-// every step), which otherwise costs as much LDS bandwidth as the MFMAs take time.
 // TL: the codes come from the matrix's 128-row tile-major copy (5-bit): a K step of 128 rows
 // is one contiguous 5,120-byte block, so each dword copy instruction of a wave reads 256
 // contiguous bytes instead of pieces of six or seven rows 1,280 bytes apart.
@@ -385,17 +383,22 @@ constexpr int qmm_lds_occupancy() {
 // copies fill (slots past NTC tiles repeat the chunk's first route and are not multiplied):
 // 96-route chunks for the 5-bit gated launches of config-4-like routing, where no expert
 // then needs a second chunk.
-template <int BITS, bool GATED, int NT, int S, bool SPLIT, int RS = 1, bool TL = false, int NTC = NT>
-__global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<BITS, GATED, NT, SPLIT>())) void qmm_lds_kernel(QmmParams P) {
+// KS: K steps per unrolled window. 8 loads a row's scales 16 bytes at a time; 4 (dense
+// only) lets a launch split K in ranges of whole four-step windows (P.ksplit ranges of
+// P.ksteps steps, the last one shorter), each range a work item of its own. With several
+// ranges y is the planes' buffer: a block stores its f32 accumulators as they lie in
+// registers (1 KB a store instruction, where the tokens' rows would be 16-byte pieces) at its
+// (row tile, chunk) place of plane `range`, and splitk_sum_kernel adds the planes up.
+template <int BITS, bool GATED, int NT, int S, bool SPLIT, bool TL = false, int NTC = NT, int KS = 8>
+__global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_occupancy<BITS, GATED, NT, SPLIT>())) void qmm_lds_kernel(QmmParams P) {
     // 32-route tiles (NT = 1) serve the 8-bit grouped down projection of sparse routing only
     // (gate/up measured slower: config 3 181 -> 247 us). Their earlier wrong results, like
     // other schedule-dependent failures of this kernel, came from MFMAs reading bf16 operands
     // converted by inline asm one instruction earlier; the conversion is now visible to the
     // compiler.
     static_assert(!SPLIT || GATED, "only the gated kernel splits its matrices over waves");
-    static_assert(RS == 1 || (!GATED && !SPLIT), "two slabs a wave: non-gated only");
     static_assert(!TL || BITS == 5, "tile-major codes: 5-bit only");
-    constexpr int TR = 128 * RS;             // rows per row tile
+    constexpr int TR = 128;                  // rows per row tile
     constexpr int NW = SPLIT ? 8 : 4;        // waves per block
     static_assert(NTC >= 1 && NTC <= NT, "compute tiles within the copied route slots");
     constexpr int BN = 32 * NTC;             // routes per chunk (multiplied)
@@ -406,7 +409,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
     constexpr int WMAT = SPLIT ? 1 : NMAT;   // matrices one wave dequantizes
     constexpr int B_ST = BC * 128;
     constexpr int ST = NMAT * A_ST + B_ST;   // bytes per stage
-    constexpr int AQ = (BITS == 8 ? 2 : 5) * RS;   // direct copies per wave per matrix per step
+    constexpr int AQ = BITS == 8 ? 2 : 5;   // direct copies per wave per matrix per step
     constexpr int NBW = 4 * NT / NW;         // activation copies (8 routes each) per wave
     static_assert(NBW >= 1 && NBW * NW == 4 * NT, "activation pieces split evenly over the waves");
     constexpr int LPS = WMAT * AQ + NBW;     // copies per thread per step
@@ -419,7 +422,11 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
     // split: silu(gate) of XNT route tiles at a time (in halves when four tiles would not fit
     // beside the stages)
     constexpr int XNT = SPLIT && NTC > 3 ? NTC / 2 : NTC;
-    __shared__ __align__(16) float xch[SPLIT ? 4 * XNT * 16 * 64 : 1];
+    float *xch = nullptr;
+    if constexpr (SPLIT) {
+        __shared__ __align__(16) float xbuf[4 * XNT * 16 * 64];
+        xch = xbuf;
+    }
     lds_escape(st0, st1, st2, st3, xch);
     auto stage_base = [&](int stage) -> unsigned char * {
         return stage == 0 ? st0 : stage == 1 ? st1 : stage == 2 ? st2 : st3;
@@ -432,8 +439,17 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
     // ---- work item (every wave derives it): physical block b runs logical item
     // L = xcd_item(b, items); L = chunk * rt_groups + row-tile group, a group being up to
     // rtb consecutive row tiles
-    int e = 0, first = 0, nvalid = 0, rt0 = -1, nrt = 0;
-    {
+    static_assert(KS == 8 || (KS == 4 && !GATED && NT == NTC), "K ranges: dense launches only");
+    int e = 0, first = 0, nvalid = 0, rt0 = -1, nrt = 0, range = 0;
+    if constexpr (KS == 4) {
+        // grid (row tile, K range, chunk): no index is divided on the way to the first copies;
+        // a row tile's chunks meet on one XCD when the row tiles are a multiple of eight
+        rt0 = (int)blockIdx.x;
+        nrt = 1;
+        range = (int)blockIdx.y;
+        first = (int)blockIdx.z * BN;
+        nvalid = min(BN, P.tokens - first);
+    } else {
         const int chunks = P.dense ? (P.tokens + BN - 1) / BN : chunk_total<BN>(P.counts, P.ngroups);
         const int L = xcd_item((int)blockIdx.x, chunks * P.rt_groups);
         const int ci = L < 0 ? chunks : L / P.rt_groups;
@@ -462,14 +478,17 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
     nrt = __builtin_amdgcn_readfirstlane(nrt);
     if (rt0 < 0) return;
     const int C = P.columns, R = P.rows, G = C >> 6;
+    // this block's K steps: k0 .. k0 + NK - 1
+    const int k0 = KS == 4 ? range * P.ksteps : 0;
+    const int NK = KS == 4 ? min(P.ksteps, G - k0) : G;
     // route of the chunk's n-th slot (slots past the chunk repeat its first route)
     auto route_at = [&](int n) -> int {
         n = n < nvalid ? n : 0;
-        return P.dense ? first + n : (int)P.routes[(size_t)e * P.tokens + first + n];
+        return KS == 4 || P.dense ? first + n : (int)P.routes[(size_t)e * P.tokens + first + n];
     };
 
     // ---- weights
-    const bool shared = !P.dense && e == P.experts;
+    const bool shared = KS != 4 && !P.dense && e == P.experts;
     const char *pw[2] = {reinterpret_cast<const char *>(shared ? P.sp0 : P.p0),
                          reinterpret_cast<const char *>(shared ? P.sp1 : P.p1)};
     const uint16_t *psc[2] = {shared ? P.ss0 : P.s0, shared ? P.ss1 : P.s1};
@@ -486,31 +505,29 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
     for (int q = 0; q < AQ; q++) {
         if constexpr (BITS == 8) {
             const int rl = 16 * q + (lane >> 2), sl = lane & 3;
-            crow[q] = slab * 32 * RS + rl;
+            crow[q] = slab * 32 + rl;
             coff[q] = 16 * (sl ^ ((rl >> 2) & 3));
         } else {
             const int i = 64 * q + lane, rl = i / 10;
-            crow[q] = slab * 32 * RS + rl;
+            crow[q] = slab * 32 + rl;
             coff[q] = 4 * (i - rl * 10);
         }
     }
     // this lane's MFMA row; its scale/bias bf16 bits come eight groups per 16-byte load
     const int r = lane & 31, h = lane >> 5;
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    typedef unsigned int wvec __attribute__((ext_vector_type(KS / 2)));   // a window's scales
     // The loads go through global-address-space pointers: with the matrix picked by the wave
     // (split form) the compiler cannot tell the generic pointer is global, emits FLAT loads,
     // and a FLAT load may read LDS, so it first waits for every LDS copy in flight (a full
     // drain of the copy pipeline once per eight steps).
-    typedef __attribute__((address_space(1))) const u32x4 g_u32x4;
-    auto win_load = [&](u32x4 (&sw)[RS][2][2], int ti, int w) {
+    typedef __attribute__((address_space(1))) const wvec g_wvec;
+    auto win_load = [&](wvec (&sw)[2][2], int ti, int w) {
+        const size_t mrow = row_index(rt0 + ti, slab * 32 + r);
 #pragma unroll
-        for (int rs = 0; rs < RS; rs++) {
-            const size_t mrow = row_index(rt0 + ti, slab * 32 * RS + 32 * rs + r);
-#pragma unroll
-            for (int m = 0; m < WMAT; m++) {
-                sw[rs][m][0] = *(g_u32x4 *)(psc[m + mw] + mrow * G + 8 * w);
-                sw[rs][m][1] = *(g_u32x4 *)(pbi[m + mw] + mrow * G + 8 * w);
-            }
+        for (int m = 0; m < WMAT; m++) {
+            sw[m][0] = *(g_wvec *)(psc[m + mw] + mrow * G + k0 + KS * w);
+            sw[m][1] = *(g_wvec *)(pbi[m + mw] + mrow * G + k0 + KS * w);
         }
     };
 
@@ -521,8 +538,8 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
     for (int i = 0; i < NBW; i++) {
         const int n = (NW * i + wave) * 8 + (lane >> 3), sl = lane & 7;
         const int route = route_at(n);
-        const int in_row = P.in_mode == 1 ? (route < T8 ? (route >> 3) : route - T8) : route;
-        bsrc[i] = P.x + (size_t)in_row * C + 8 * (sl ^ ((n >> 1) & 7));
+        const int in_row = KS != 4 && P.in_mode == 1 ? (route < T8 ? (route >> 3) : route - T8) : route;
+        bsrc[i] = P.x + (size_t)in_row * C + 64 * k0 + 8 * (sl ^ ((n >> 1) & 7));
     }
     // output routes of this lane's accumulator columns
     int out_route[NTC];
@@ -545,7 +562,8 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
     const size_t wrows = TL ? (size_t)((R + 255) & ~255) : (size_t)R;  // code rows per expert
     const char *wbase[WMAT];
 #pragma unroll
-    for (int mm = 0; mm < WMAT; mm++) wbase[mm] = pw[mm + mw] + (size_t)(shared ? 0 : e) * wrows * row_bytes;
+    for (int mm = 0; mm < WMAT; mm++)
+        wbase[mm] = pw[mm + mw] + (size_t)(shared ? 0 : e) * wrows * row_bytes + (size_t)k0 * KSTEP;
     // Tile-major: the lane's offset within a row tile's first K step is fixed, and a tile adds
     // the wave-uniform tile * TR * row_bytes. No clamp: an expert's last tile reads zero
     // padding rows (in bounds; their outputs are not stored). Held so, the 5-bit kernels spend
@@ -590,14 +608,14 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
             for (int q = 0; q < AQ; q++) {
                 const char *src = wbase[mm] + (woff[q] + koff);
                 if constexpr (BITS == 8)
-                    to_lds<16>(src, base + m * A_ST + (slab * 32 * RS + 16 * q) * 64);
+                    to_lds<16>(src, base + m * A_ST + (slab * 32 + 16 * q) * 64);
                 else
-                    to_lds<4>(src, base + m * A_ST + slab * 32 * RS * 40 + q * 256);
+                    to_lds<4>(src, base + m * A_ST + slab * 32 * 40 + q * 256);
             }
         }
 #pragma unroll
         for (int i = 0; i < NBW; i++) to_lds<16>(bsrc[i] + 64 * iss_kg, base + NMAT * A_ST + (NW * i + wave) * 8 * 128);
-        if (iss_kg + 1 < G) {
+        if (iss_kg + 1 < NK) {
             iss_kg++;
         } else if (iss_ti + 1 < nrt) {
             iss_ti++;
@@ -605,20 +623,19 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
         }
     };
 
+    wvec win[2][2], win_next[2][2];
+    if constexpr (KS == 4) win_load(win, 0, 0);   // (few steps: the first must not wait for the third's copies)
 #pragma unroll
     for (int st = 0; st < S - 1; st++) issue(st);
-    u32x4 win[RS][2][2], win_next[RS][2][2];
-    win_load(win, 0, 0);
+    if constexpr (KS != 4) win_load(win, 0, 0);
 
-    dih_f32x16 acc0[RS][NTC], acc1[GATED && !SPLIT ? NTC : 1];
+    dih_f32x16 acc0[NTC], acc1[GATED && !SPLIT ? NTC : 1];
     auto zero_acc = [&]() {
 #pragma unroll
-        for (int rs = 0; rs < RS; rs++)
+        for (int i = 0; i < NTC; i++) {
 #pragma unroll
-            for (int i = 0; i < NTC; i++) {
-#pragma unroll
-                for (int k = 0; k < 16; k++) acc0[rs][i][k] = 0.f;
-            }
+            for (int k = 0; k < 16; k++) acc0[i][k] = 0.f;
+        }
         if constexpr (GATED && !SPLIT) {
 #pragma unroll
             for (int i = 0; i < NTC; i++) {
@@ -632,24 +649,22 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
     auto run = [&](auto ntu_c) {
     constexpr int NTU = decltype(ntu_c)::value;
     for (int ti = 0; ti < nrt; ti++) {
-        for (int kw = 0; kw < G; kw += 8) {
+        for (int kw = 0; kw < NK; kw += KS) {
             // the next window of scales: this tile's next one, or the next tile's first
-            const bool more = kw + 8 < G || ti + 1 < nrt;
-            if (more) win_load(win_next, kw + 8 < G ? ti : ti + 1, kw + 8 < G ? (kw >> 3) + 1 : 0);
+            const bool more = kw + KS < NK || ti + 1 < nrt;
+            if (more) win_load(win_next, kw + KS < NK ? ti : ti + 1, kw + KS < NK ? kw / KS + 1 : 0);
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
+            for (int u = 0; u < KS; u++) {
                 wait_vm<(S - 2) * LPS>();
                 barrier_no_fence();
                 issue((u + S - 1) % S);
                 const unsigned char *base = stage_base(u % S);
-                // this step's weights -> bf16 A operands (a[rs * WMAT + m]: slab rs, matrix m)
-                dih_bf16x8 a[RS * 2][4];
-#pragma unroll
-                for (int rs = 0; rs < RS; rs++)
+                // this step's weights -> bf16 A operands
+                dih_bf16x8 a[2][4];
 #pragma unroll
                 for (int m = 0; m < WMAT; m++) {
                     Chunk<BITS> c;
-                    const int wr = slab * 32 * RS + 32 * rs + r;   // row within the tile
+                    const int wr = slab * 32 + r;   // row within the tile
                     if constexpr (BITS == 8) {
                         const int sw = (r >> 2) & 3;
                         const unsigned char *ra = base + (m + mw) * A_ST + wr * 64;
@@ -662,9 +677,9 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
 #pragma unroll
                         for (int k = 0; k < 5; k++) c.w[k] = ra[k];
                     }
-                    const uint32_t sbits = (win[rs][m][0][u >> 1] >> (16 * (u & 1))) & 0xffffu;
-                    const uint32_t bbits = (win[rs][m][1][u >> 1] >> (16 * (u & 1))) & 0xffffu;
-                    chunk_to_bf16<BITS>(c, bf16_to_f32(sbits), bf16_to_f32(bbits), a[rs * WMAT + m]);
+                    const uint32_t sbits = (win[m][0][u >> 1] >> (16 * (u & 1))) & 0xffffu;
+                    const uint32_t bbits = (win[m][1][u >> 1] >> (16 * (u & 1))) & 0xffffu;
+                    chunk_to_bf16<BITS>(c, bf16_to_f32(sbits), bf16_to_f32(bbits), a[m]);
                 }
                 // MFMAs over all NT route tiles
                 const unsigned char *bb = base + NMAT * A_ST;
@@ -678,9 +693,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
                     }
 #pragma unroll
                     for (int i = 0; i < NTU; i++) {
-#pragma unroll
-                        for (int rs = 0; rs < RS; rs++)
-                            acc0[rs][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[rs * WMAT][j], bx[i], acc0[rs][i], 0, 0, 0);
+                        acc0[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][j], bx[i], acc0[i], 0, 0, 0);
                         if constexpr (GATED && !SPLIT)
                             acc1[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][j], bx[i], acc1[i], 0, 0, 0);
                     }
@@ -688,9 +701,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
             }
             if (more) {
 #pragma unroll
-                for (int rs = 0; rs < RS; rs++)
-#pragma unroll
-                    for (int m = 0; m < WMAT; m++) { win[rs][m][0] = win_next[rs][m][0]; win[rs][m][1] = win_next[rs][m][1]; }
+                for (int m = 0; m < WMAT; m++) { win[m][0] = win_next[m][0]; win[m][1] = win_next[m][1]; }
             }
         }
 
@@ -700,6 +711,21 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
         // time; the up waves store.
 #pragma unroll
         for (int half = 0; half < NTC / XNT; half++) {
+        if constexpr (KS == 4) {
+            if (P.ksplit > 1) {
+                const size_t at = ((size_t)(range * gridDim.x + rt0) * gridDim.z + blockIdx.z) * (TR * BN);
+                dih_f32x4 *dst = reinterpret_cast<dih_f32x4 *>(static_cast<float *>(P.y) + at) + slab * (NTC * 4 * 64) + lane;
+#pragma unroll
+                for (int i = 0; i < NTC; i++) {
+                    if (32 * i >= nvalid) break;
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        dst[(i * 4 + q) * 64] = dih_f32x4{acc0[i][4 * q], acc0[i][4 * q + 1], acc0[i][4 * q + 2],
+                                                          acc0[i][4 * q + 3]};
+                }
+                break;
+            }
+        }
         if constexpr (SPLIT) {
             if (half > 0) {   // the up waves have read the previous half
                 wait_lgkm0();
@@ -710,15 +736,13 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
 #pragma unroll
                 for (int i = 0; i < XNT; i++) {
 #pragma unroll
-                    for (int k = 0; k < 16; k++) xw[(i * 16 + k) * 64] = siluf_(acc0[0][half * XNT + i][k]);
+                    for (int k = 0; k < 16; k++) xw[(i * 16 + k) * 64] = siluf_(acc0[half * XNT + i][k]);
                 }
             }
             wait_lgkm0();
             barrier_no_fence();
         }
-#pragma unroll
-        for (int rs = 0; rs < RS; rs++) {
-        const int row_base = (rt0 + ti) * TR + slab * 32 * RS + 32 * rs;
+        const int row_base = (rt0 + ti) * TR + slab * 32;
 #pragma unroll
         for (int ii = 0; ii < XNT; ii++) {
             const int i = half * XNT + ii;
@@ -731,7 +755,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
                 float v[4];
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
-                    const float g = acc0[rs][i][4 * q + k];
+                    const float g = acc0[i][4 * q + k];
                     if constexpr (SPLIT) v[k] = xch[(slab * XNT * 16 + ii * 16 + 4 * q + k) * 64 + lane] * g;
                     else if constexpr (GATED) v[k] = siluf_(g) * acc1[i][4 * q + k];
                     else v[k] = g;
@@ -756,7 +780,6 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (RS > 1 ? 1 : qmm_lds_occupancy<
                     }
                 }
             }
-        }
         }
         }
         zero_acc();
@@ -806,10 +829,55 @@ bool matrix_retile(Matrix *m, size_t first, size_t count, char *error, int capac
            hip_ok(hipStreamSynchronize(nullptr), error, capacity, "weight retile");
 }
 
+// The planes of a split-K dense launch summed in range order, one accumulator quad (four
+// rows of one token) a thread: quad f of a plane is lane f % 64, rows 8q + 4 (lane / 32) ..
+// of 32-row slab w, token 32i + lane % 32, for f / 64 = ((item * 4 + w) * nt + i) * 4 + q and
+// item = row tile * chunks + chunk. Latency-bound: a thread's planes are requested sixteen at
+// a time.
+__global__ __launch_bounds__(256) void splitk_sum_kernel(const dih_f32x4 *__restrict__ part, size_t quads, int planes,
+                                                         int nt, int chunks, int T, int R, void *__restrict__ y,
+                                                         int y_bf16) {
+    const size_t f = (size_t)blockIdx.x * 256 + threadIdx.x;   // (quads is a multiple of 256)
+    const int lane = (int)(f & 63);
+    int g = (int)(f >> 6);
+    const int q = g & 3;
+    g >>= 2;
+    const int i = g % nt;
+    g /= nt;
+    const int w = g & 3, item = g >> 2, rt = item / chunks, chunk = item - rt * chunks;
+    const int tok = (chunk * nt + i) * 32 + (lane & 31), row = rt * 128 + w * 32 + 8 * q + 4 * (lane >> 5);
+    if (tok >= T || row >= R) return;
+    dih_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < planes; s += 16) {
+        dih_f32x4 v[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++)
+            if (s + k < planes) v[k] = part[(size_t)(s + k) * quads + f];
+#pragma unroll
+        for (int k = 0; k < 16; k++)
+            if (s + k < planes) acc += v[k];
+    }
+    const size_t o = (size_t)tok * R + row;
+    if ((R & 3) == 0) {   // (rows of whole quads, as the unsplit kernel stores them)
+        if (y_bf16)
+            *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(y) + o) =
+                uint2{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
+        else
+            *reinterpret_cast<dih_f32x4 *>(static_cast<float *>(y) + o) = acc;
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (row + k >= R) break;
+            if (y_bf16) static_cast<uint16_t *>(y)[o + k] = f32_to_bf16(acc[k]);
+            else static_cast<float *>(y)[o + k] = acc[k];
+        }
+    }
+}
+
 // Upper bound of (row tile, chunk) work items: sum_g ceil(count_g / BN) <= routes / BN +
 // (groups holding any route); a shared-expert group adds `tokens` routes.
-static size_t qmm_max_work(int rows, int tokens, int ngroups, int dense, int bn, int tile_rows = 128) {
-    const size_t row_tiles = (size_t)(rows + tile_rows - 1) / tile_rows;
+static size_t qmm_max_work(int rows, int tokens, int ngroups, int dense, int bn) {
+    const size_t row_tiles = (size_t)(rows + 127) / 128;
     if (dense) return row_tiles * ((size_t)(tokens + bn - 1) / bn);
     const size_t routes = (size_t)tokens * 9;
     return row_tiles * (routes / bn + std::min<size_t>((size_t)ngroups, routes));
@@ -818,6 +886,123 @@ static size_t qmm_max_work(int rows, int tokens, int ngroups, int dense, int bn,
 bool qmm_wide_gated(const Matrix *gate, int tokens) {
     return gate->bits == 5 && gate->columns % 512 == 0 &&
            (size_t)tokens * 8 > (size_t)48 * (size_t)std::max(1, gate->experts);
+}
+
+// The estimate dense_plan minimizes, in us, fitted to 770 measured launches (four model
+// projections, 5 and 8 bits, 16 to 1023 tokens; median error 5 %, and the plan it picks is
+// 0.5 % behind the best one on average, 7 % at worst). n blocks of nt 32-token tiles run on
+// each CU, `resident` at a time; a K step of c resident blocks takes the larger of one
+// block's latency and c times its issue time. Ranges add the sum pass: its launch and the
+// planes' write and read.
+static double dense_cost(int bits, size_t items, int nt, int steps, int ksplit, size_t plane_bytes) {
+    constexpr int kResident[2][5] = {{0, 4, 3, 2, 1}, {0, 3, 2, 2, 1}};   // by LDS: 5-bit, 8-bit
+    const int resident = kResident[bits == 8][nt];
+    const double slow = bits == 8 ? 1.0 : 1.1, latency = 0.2 + 0.111 * nt, issue = 0.185 + 0.054 * nt;
+    const size_t n = (items * (size_t)ksplit + 255) / 256;
+    const auto round = [&](size_t c) { return 0.755 + slow * steps * std::max(latency, issue * (double)c); };
+    double t = 4.3 + (double)(n / resident) * round(resident);
+    if (n % resident) t += round(n % resident);
+    return ksplit > 1 ? t + 0.78 + (double)ksplit * (double)plane_bytes * 2.0 / 5.0e6 : t;
+}
+
+// The same for one dequantization pass and the bf16 GEMM of gemm.hip: a round of 256 tiles
+// costs its shape's time a 64-column step, a partial one 60 % of that plus its share.
+static double dense_gemm_cost(const Matrix *m, int tokens) {
+    int bm, bn;
+    gemm_tile(m->rows, tokens, bm, bn);
+    const double step = bm * bn >= 65536 ? 1.77 : bm * bn >= 32768 ? 1.1 : bm * bn >= 16384 ? 0.53 : 0.37;
+    const size_t tiles = (size_t)((m->rows + bm - 1) / bm) * (size_t)((tokens + bn - 1) / bn);
+    double rounds = (double)(tiles / 256);
+    if (tiles % 256) rounds += tiles < 256 ? 1.0 : 0.6 + 0.4 * (double)(tiles % 256) / 256.0;
+    return 6.0 + (double)m->rows * m->columns * (m->bits / 8.0 + 2.0) / 5.3e6 + rounds * (m->columns / 64) * step;
+}
+
+// Limits of the kernels' 32-bit offsets: an expert's weight rows (padded to whole 256-row
+// tiles in the tile-major copy), input rows.
+static bool qmm_in_range(const Matrix *m, int tokens) {
+    return m->tiled_rows() * ((size_t)m->columns * m->bits / 8) <= 0x7fffffffu &&
+           (size_t)tokens * 9 * (size_t)m->columns <= 0x7fffffffu;
+}
+
+// Short chunks gain from ranges (61 tokens of a 2048 x 4096 8-bit matrix, 16 row tiles:
+// 31.0 us unsplit in 128-token tiles, 10.7 us in 8 ranges), the rest from narrower token
+// tiles whose blocks share a CU, so that one's dequantization overlaps another's MFMAs and
+// the last round is finer (8192 x 2048: 128 tokens 23.7 -> 13.7 us, 700 tokens 48.1 -> 29.7
+// us; 512 x 2048 at 1023 tokens 17.6 us as a GEMM -> 12.6 us).
+DensePlan dense_plan(const Matrix *m, int tokens, size_t part_bytes) {
+    DensePlan best;
+    // (shorter chunks never need the bf16 copy of the weights)
+    const bool may_gemm = tokens >= 1024 || (tokens >= 512 && m->rows <= 4096);
+    if (m->columns % 512 != 0 || !qmm_in_range(m, tokens)) {
+        best.gemm = may_gemm;
+        return best;
+    }
+    const size_t row_tiles = (size_t)(m->rows + 127) / 128;
+    const int windows = m->columns / 256;   // of four K steps
+    double cost = 0;
+    for (int nt = 1; nt <= 4; nt++) {
+        const size_t chunks = ((size_t)tokens + 32 * nt - 1) / (32 * nt), items = row_tiles * chunks;
+        const size_t plane = items * 128 * 32 * (size_t)nt * 4;
+        if (chunks > 0xffff || (nt > 1 && tokens <= 32 * (nt - 1))) continue;
+        for (int k = 1; k <= windows && (k == 1 || k * plane <= part_bytes); k *= 2) {
+            const double c = dense_cost(m->bits, items, nt, 4 * ((windows + k - 1) / k), k, plane);
+            if (best.nt == 0 || c < cost) {
+                cost = c;
+                best.nt = nt;
+                best.ksplit = k;
+            }
+        }
+    }
+    // (5 % for the estimates' error: 2048 tokens of a 2048 x 4096 matrix take 44.4 us as a GEMM
+    // and 46.9 us fused, 1300 tokens 53.6 and 36.3 us)
+    best.gemm = may_gemm && (best.nt == 0 || dense_gemm_cost(m, tokens) < 1.05 * cost);
+    return best;
+}
+
+// A dense streaming launch as planned: nt 32-token tiles a block, K in ksplit ranges.
+static bool launch_dense_split(const QmmArgs &a, QmmParams P, hipStream_t s, char *error, int capacity) {
+    const Matrix *m = a.m0;
+    const int G = m->columns >> 6, nt = a.plan.nt, chunks = (a.tokens + 32 * nt - 1) / (32 * nt);
+    P.ksteps = 4 * ((G / 4 + a.plan.ksplit - 1) / a.plan.ksplit);
+    P.ksplit = (G + P.ksteps - 1) / P.ksteps;   // (no empty range)
+    P.rtb = 1;
+    P.rt_groups = P.row_tiles;
+    const size_t quads = (size_t)P.row_tiles * chunks * (128 * 32 / 4) * nt;   // of one plane
+    if (P.ksplit > 1) {
+        if (!a.part || (size_t)P.ksplit * quads * 16 > a.part_bytes) {
+            set_error(error, capacity, "Split-K planes too small");
+            return false;
+        }
+        P.y = a.part;
+        P.y_bf16 = 0;
+    }
+    if (m->bits == 5) {
+        if (!m->tiled) {
+            set_error(error, capacity, "Missing tile-major 5-bit codes");
+            return false;
+        }
+        P.p0 = static_cast<const uint32_t *>(m->tiled);
+    }
+    const dim3 grid((unsigned)P.row_tiles, (unsigned)P.ksplit, (unsigned)chunks);
+    bool found = false;
+#define DIH_DENSE_CASE(B, N)                                                                           \
+    if (m->bits == B && nt == N) {                                                                     \
+        DIH_LAUNCH((qmm_lds_kernel<B, false, N, 4, false, B == 5, N, 4>), grid, dim3(256), 0, s, P);   \
+        found = true;                                                                                  \
+    }
+    DIH_DENSE_CASE(8, 1) DIH_DENSE_CASE(8, 2) DIH_DENSE_CASE(8, 3) DIH_DENSE_CASE(8, 4)
+    DIH_DENSE_CASE(5, 1) DIH_DENSE_CASE(5, 2) DIH_DENSE_CASE(5, 3) DIH_DENSE_CASE(5, 4)
+#undef DIH_DENSE_CASE
+    if (!found) {
+        set_error(error, capacity, "Unsupported qmm configuration");
+        return false;
+    }
+    if (!hip_ok(hipGetLastError(), error, capacity, "qmm launch")) return false;
+    if (P.ksplit == 1) return true;
+    DIH_LAUNCH(splitk_sum_kernel, dim3((unsigned)(quads / 256)), dim3(256), 0, s,
+               reinterpret_cast<const dih_f32x4 *>(a.part), quads, P.ksplit, nt, chunks, a.tokens, m->rows, a.y,
+               a.y_bf16);
+    return hip_ok(hipGetLastError(), error, capacity, "split-K sum launch");
 }
 
 bool launch_qmm(const QmmArgs &a, hipStream_t s, char *error, int capacity) {
@@ -837,15 +1022,10 @@ bool launch_qmm(const QmmArgs &a, hipStream_t s, char *error, int capacity) {
         set_error(error, capacity, "Invalid grouped qmm arguments");
         return false;
     }
-    // the streaming kernel addresses an expert's weight rows (padded to whole 256-row tiles
-    // in the tile-major copy) with 32-bit offsets
-    if (m0->tiled_rows() * ((size_t)m0->columns * m0->bits / 8) > 0x7fffffffu) {
-        set_error(error, capacity, "Matrix too large for one grouped/dense qmm launch");
-        return false;
-    }
-    // input row offsets (row * columns) are 32-bit in the kernel
-    if ((size_t)a.tokens * 9 * (size_t)m0->columns > 0x7fffffffu) {
-        set_error(error, capacity, "Chunk too large for one grouped/dense qmm launch");
+    if (!qmm_in_range(m0, a.tokens)) {
+        set_error(error, capacity, m0->tiled_rows() * ((size_t)m0->columns * m0->bits / 8) > 0x7fffffffu
+                                       ? "Matrix too large for one grouped/dense qmm launch"
+                                       : "Chunk too large for one grouped/dense qmm launch");
         return false;
     }
     // Route tile width: 64 routes for the gated kernels, 128 otherwise (the register-ring
@@ -869,19 +1049,14 @@ bool launch_qmm(const QmmArgs &a, hipStream_t s, char *error, int capacity) {
                            (size_t)a.tokens * 8 > (size_t)48 * (size_t)std::max(1, m0->experts);
     const bool narrow_down = streaming && !gated && !a.dense && m0->bits == 8 &&
                              (size_t)a.tokens * 8 <= (size_t)16 * (size_t)std::max(1, m0->experts);
+    if (streaming && a.dense && !gated) return launch_dense_split(a, P, s, error, capacity);
     const int nt = streaming && !a.dense && !gated ? (wide_down ? 3 : narrow_down ? 1 : 2)
                                                    : (gated ? (wide_gated ? 4 : 2) : 4);
     // wide 5-bit gated chunks of 96 routes when experts average at most 64 routes (the copies
     // still fill 128 route slots; the MFMAs cover 96)
     const int ntc = wide_gated && (size_t)a.tokens * 8 <= (size_t)64 * (size_t)std::max(1, m0->experts) ? 3 : nt;
     const int bn = 32 * ntc;
-    // dense streaming GEMMs with enough (256-row tile, route chunk) items to fill the GPU:
-    // two 32-row slabs per wave (256-row tiles)
-    const bool two_slabs = streaming && a.dense && !gated &&
-                           (size_t)((m0->rows + 255) / 256) * (size_t)((a.tokens + bn - 1) / bn) >= 256;
-    const int tile_rows = two_slabs ? 256 : 128;
-    P.row_tiles = (m0->rows + tile_rows - 1) / tile_rows;
-    const size_t work = qmm_max_work(m0->rows, a.tokens, a.ngroups, a.dense, bn, tile_rows);
+    const size_t work = qmm_max_work(m0->rows, a.tokens, a.ngroups, a.dense, bn);
     const size_t blocks = 8 * ((work + 7) / 8);
     if (blocks == 0 || blocks > 0x7fffffffu) {
         set_error(error, capacity, "Invalid qmm grid");
@@ -923,16 +1098,15 @@ bool launch_qmm(const QmmArgs &a, hipStream_t s, char *error, int capacity) {
         // Gated launches: the split eight-wave form (gate and up on different waves, so one
         // wave's dequant overlaps the other's MFMAs and waits): 6 % faster on config 4, and,
         // since empty route tiles are skipped, config 3 gate/up 154 -> 143 us
-#define DIH_QMM_LDS_CASE(B, GT, N, R2, NC)                                          \
-        if (m0->bits == B && gated == GT && nt == N && two_slabs == R2 && ntc == NC) { \
+#define DIH_QMM_LDS_CASE(B, GT, N, NC)                                              \
+        if (m0->bits == B && gated == GT && nt == N && ntc == NC) {                 \
             constexpr bool SP = GT;                                                 \
-            DIH_LAUNCH((qmm_lds_kernel<B, GT, N, 4, SP, R2 ? 2 : 1, B == 5, NC>), grid, dim3(SP ? 512 : 256), 0, s, P); \
+            DIH_LAUNCH((qmm_lds_kernel<B, GT, N, 4, SP, B == 5, NC>), grid, dim3(SP ? 512 : 256), 0, s, P); \
             return hip_ok(hipGetLastError(), error, capacity, "qmm launch");        \
         }
-        DIH_QMM_LDS_CASE(8, true, 2, false, 2) DIH_QMM_LDS_CASE(8, false, 2, false, 2) DIH_QMM_LDS_CASE(8, false, 1, false, 1) DIH_QMM_LDS_CASE(8, false, 4, false, 4)
-        DIH_QMM_LDS_CASE(5, true, 2, false, 2) DIH_QMM_LDS_CASE(5, false, 2, false, 2) DIH_QMM_LDS_CASE(5, false, 3, false, 3) DIH_QMM_LDS_CASE(5, false, 4, false, 4)
-        DIH_QMM_LDS_CASE(5, true, 4, false, 4) DIH_QMM_LDS_CASE(5, true, 4, false, 3)
-        DIH_QMM_LDS_CASE(8, false, 4, true, 4) DIH_QMM_LDS_CASE(5, false, 4, true, 4)
+        DIH_QMM_LDS_CASE(8, true, 2, 2) DIH_QMM_LDS_CASE(8, false, 2, 2) DIH_QMM_LDS_CASE(8, false, 1, 1)
+        DIH_QMM_LDS_CASE(5, true, 2, 2) DIH_QMM_LDS_CASE(5, false, 2, 2) DIH_QMM_LDS_CASE(5, false, 3, 3)
+        DIH_QMM_LDS_CASE(5, true, 4, 4) DIH_QMM_LDS_CASE(5, true, 4, 3)
 #undef DIH_QMM_LDS_CASE
     }
 #define DIH_QMM_CASE(B, GT, N, D)                                                   \

@@ -775,6 +775,74 @@ def test_dense_two_slab_tiles(device, bits, rows, columns, T):
         m.dispose()
 
 
+@pytest.mark.parametrize("bits", [8, 5])
+@pytest.mark.parametrize("rows,columns,T", [
+    (512, 2048, 5), (512, 2048, 32), (2048, 4096, 33), (2048, 4096, 64), (300, 2048, 65), (129, 4096, 96),
+    (1003, 2048, 97), (2048, 512, 128), (513, 1536, 129), (4100, 512, 160), (512, 8192, 193), (300, 2560, 300),
+    (8192, 512, 700), (512, 2048, 1300), (2048, 1024, 1500)])   # (the last two past the GEMM's first token count)
+def test_dense_split_ranges(device, bits, rows, columns, T):
+    """Short dense chunks split K over work items and sum the planes: one to four 32-token
+    tiles a block, one and several ranges (the last one shorter: 1536 and 2560 columns), rows
+    past and off the 128-row tiles, rows not whole float4. f32 within fp32 accumulation of the
+    product of bf16-rounded operands, bf16 the same answer rounded once."""
+    rng = np.random.default_rng(rows + columns + T)
+    host = orc.random_matrix(rng, 1, rows, columns, bits)
+    m = upload(device, host)
+    try:
+        xb = orc.f32_to_bf16_bits(rng.normal(size=(T, columns)).astype(np.float32))
+        y = torch.full((T + 1, rows), 7.0, dtype=torch.float32, device="cuda")
+        yb = torch.full((T + 1, rows), 7, dtype=torch.int16, device="cuda")
+        dh.dense(device, m, T, dev_bf16(xb), y)
+        dh.dense(device, m, T, dev_bf16(xb), yb, y_dtype=dh.BF16)
+        torch.cuda.synchronize()
+        got = y.cpu().numpy()
+        want = orc.dense_f64_blas(host, orc.bf16_bits_to_f32(xb), round_operands=True)
+        assert orc.rel_err(got[:T], want) < 1e-4
+        assert np.array_equal(yb[:T].cpu().numpy().view(np.uint16), orc.f32_to_bf16_bits(got[:T]))
+        assert (got[T] == 7.0).all() and (yb[T].cpu().numpy() == 7).all()
+    finally:
+        m.dispose()
+
+
+def test_dense_short_chunks_on_streams_and_in_graphs():
+    """Split-K planes belong to a stream: calls on more streams than a context holds planes
+    for (the last ones run unsplit), queued beside each other on one context, and a call
+    captured in a graph as the context's first (nothing allocated) all give the f64 product."""
+    rng = np.random.default_rng(61)
+    T, rows, columns = 61, 512, 4096
+    host = orc.random_matrix(rng, 1, rows, columns, 8)
+    xs = [orc.f32_to_bf16_bits(rng.normal(size=(T, columns)).astype(np.float32)) for _ in range(6)]
+    want = [orc.dense_f64(host, orc.bf16_bits_to_f32(x), round_operands=True) for x in xs]
+    with dh.QuantizedHip() as dev:
+        m = upload(dev, host)
+        x0 = dev_bf16(xs[0])
+        yg = torch.zeros((T, rows), device="cuda")
+        g = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g):
+            dh.dense(dev, m, T, x0, yg)
+        streams = [torch.cuda.Stream() for _ in range(6)]
+        dx = [dev_bf16(x) for x in xs]
+        ys = [torch.zeros((T, rows), device="cuda") for _ in xs]
+        torch.cuda.synchronize()
+        for rounds in range(3):
+            for y in ys:
+                y.zero_()
+            yg.zero_()
+            torch.cuda.synchronize()
+            for _ in range(4):
+                g.replay()
+                for st, x, y in zip(streams, dx, ys):
+                    with torch.cuda.stream(st):
+                        dh.dense(dev, m, T, x, y)
+            torch.cuda.synchronize()
+            for y, w in zip(ys, want):
+                assert orc.rel_err(y.cpu().numpy(), w) < 1e-4
+            assert orc.rel_err(yg.cpu().numpy(), want[0]) < 1e-4
+        del g
+        m.dispose()
+
+
 def _device_copy(dst: int, src: int, n: int) -> None:
     """hipMemcpy through the HIP runtime torch has already loaded (same soname)."""
     hip = ctypes.CDLL("libamdhip64.so.7")
