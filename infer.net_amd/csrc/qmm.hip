@@ -362,15 +362,14 @@ __global__ __launch_bounds__(256, 2) void qmm_kernel(QmmParams P) {
 
 // (to_lds, wait_vm, wait_lgkm0 and barrier_no_fence are in dih_device.h)
 
-// Blocks per CU the streaming kernel is built for: two for the narrow route tiles (two
-// 32-route tiles per matrix, three for one 5-bit matrix) when four stages fit in half the
-// LDS; the VGPR budget is then 256 per lane, accumulators included. The split gated form
-// (eight waves) runs one block.
-template <int BITS, bool GATED, int NT, bool SPLIT>
-constexpr int qmm_lds_occupancy() {
-    return !SPLIT && (GATED ? 2 : 1) * NT <= (BITS == 5 ? 3 : 2) &&
-                   4 * ((GATED ? 2 : 1) * 128 * (64 * BITS / 8) + 32 * NT * 128) <= 80 * 1024
-               ? 2 : 1;
+// Waves per SIMD the streaming kernel's registers are sized for: two blocks a CU where four
+// stages fit in half the LDS and the accumulators in the registers (four-wave blocks 256 a
+// lane, eight-wave ones 128), else one.
+template <int BITS, bool GATED, int NT, int NTC, bool SPLIT>
+constexpr int qmm_lds_waves() {
+    const bool two = 4 * ((GATED ? 2 : 1) * 128 * (64 * BITS / 8) + 32 * NT * 128) <= 80 * 1024 &&
+                     (SPLIT ? NTC <= 2 : (GATED ? 2 : 1) * NTC <= 3);
+    return (two ? 2 : 1) * (SPLIT ? 2 : 1);
 }
 
 // SPLIT (gated only): eight waves, waves 0-3 the gate matrix and 4-7 the up matrix of the
@@ -390,12 +389,7 @@ constexpr int qmm_lds_occupancy() {
 // registers (1 KB a store instruction, where the tokens' rows would be 16-byte pieces) at its
 // (row tile, chunk) place of plane `range`, and splitk_sum_kernel adds the planes up.
 template <int BITS, bool GATED, int NT, int S, bool SPLIT, bool TL = false, int NTC = NT, int KS = 8>
-__global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_occupancy<BITS, GATED, NT, SPLIT>())) void qmm_lds_kernel(QmmParams P) {
-    // 32-route tiles (NT = 1) serve the 8-bit grouped down projection of sparse routing only
-    // (gate/up measured slower: config 3 181 -> 247 us). Their earlier wrong results, like
-    // other schedule-dependent failures of this kernel, came from MFMAs reading bf16 operands
-    // converted by inline asm one instruction earlier; the conversion is now visible to the
-    // compiler.
+__global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, NTC, SPLIT>())) void qmm_lds_kernel(QmmParams P) {
     static_assert(!SPLIT || GATED, "only the gated kernel splits its matrices over waves");
     static_assert(!TL || BITS == 5, "tile-major codes: 5-bit only");
     constexpr int TR = 128;                  // rows per row tile
@@ -410,24 +404,18 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_occupancy<BITS, GATED, 
     constexpr int B_ST = BC * 128;
     constexpr int ST = NMAT * A_ST + B_ST;   // bytes per stage
     constexpr int AQ = BITS == 8 ? 2 : 5;   // direct copies per wave per matrix per step
-    constexpr int NBW = 4 * NT / NW;         // activation copies (8 routes each) per wave
-    static_assert(NBW >= 1 && NBW * NW == 4 * NT, "activation pieces split evenly over the waves");
+    constexpr int NBW = 4 * NT < NW ? 1 : 4 * NT / NW;   // activation copies (8 routes each) per wave
+    static_assert(4 * NT < NW || NBW * NW == 4 * NT, "activation pieces split evenly over the waves");
+    // (fewer pieces than waves: a piece is copied by two waves, the same bytes to the same place,
+    // which keeps every wave's outstanding copies equal)
+    constexpr int PW = 4 * NT < NW ? 4 * NT : NW;
     constexpr int LPS = WMAT * AQ + NBW;     // copies per thread per step
     static_assert(S == 4, "the stage of step s is s % 4, static within the eight-step unroll");
     // one array per stage: with the stage known at compile time the compiler can tell that an
     // operand read does not alias the copies in flight to the other stages. Nothing else
-    // lives in LDS (the split form adds the SwiGLU exchange), so that two blocks fit on a
-    // CU when the stages take half of it.
+    // lives in LDS, so that two blocks fit on a CU when the stages take half of it.
     __shared__ __align__(16) unsigned char st0[ST], st1[ST], st2[ST], st3[ST];
-    // split: silu(gate) of XNT route tiles at a time (in halves when four tiles would not fit
-    // beside the stages)
-    constexpr int XNT = SPLIT && NTC > 3 ? NTC / 2 : NTC;
-    float *xch = nullptr;
-    if constexpr (SPLIT) {
-        __shared__ __align__(16) float xbuf[4 * XNT * 16 * 64];
-        xch = xbuf;
-    }
-    lds_escape(st0, st1, st2, st3, xch);
+    lds_escape(st0, st1, st2, st3);
     auto stage_base = [&](int stage) -> unsigned char * {
         return stage == 0 ? st0 : stage == 1 ? st1 : stage == 2 ? st2 : st3;
     };
@@ -536,7 +524,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_occupancy<BITS, GATED, 
     const uint16_t *bsrc[NBW];
 #pragma unroll
     for (int i = 0; i < NBW; i++) {
-        const int n = (NW * i + wave) * 8 + (lane >> 3), sl = lane & 7;
+        const int n = (NW * i + wave % PW) * 8 + (lane >> 3), sl = lane & 7;
         const int route = route_at(n);
         const int in_row = KS != 4 && P.in_mode == 1 ? (route < T8 ? (route >> 3) : route - T8) : route;
         bsrc[i] = P.x + (size_t)in_row * C + 64 * k0 + 8 * (sl ^ ((n >> 1) & 7));
@@ -614,7 +602,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_occupancy<BITS, GATED, 
             }
         }
 #pragma unroll
-        for (int i = 0; i < NBW; i++) to_lds<16>(bsrc[i] + 64 * iss_kg, base + NMAT * A_ST + (NW * i + wave) * 8 * 128);
+        for (int i = 0; i < NBW; i++) to_lds<16>(bsrc[i] + 64 * iss_kg, base + NMAT * A_ST + (NW * i + wave % PW) * 8 * 128);
         if (iss_kg + 1 < NK) {
             iss_kg++;
         } else if (iss_ti + 1 < nrt) {
@@ -707,10 +695,9 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_occupancy<BITS, GATED, 
 
         // ---- epilogue of row tile rt0 + ti: lane holds route n = 32i + r, rows
         // 8*(k/4) + 4h + (k%4) of the slab's 32. Split: the gate waves hand silu(g) to the up
-        // waves of the same slab through LDS (identical lane layouts), XNT route tiles at a
-        // time; the up waves store.
-#pragma unroll
-        for (int half = 0; half < NTC / XNT; half++) {
+        // waves of the same slab through LDS (identical lane layouts), in the stage numbered as
+        // the slab (a gated block has one row tile, so the stages are free once every wave's
+        // copies have landed and its last operands are read); the up waves store.
         if constexpr (KS == 4) {
             if (P.ksplit > 1) {
                 const size_t at = ((size_t)(range * gridDim.x + rt0) * gridDim.z + blockIdx.z) * (TR * BN);
@@ -726,17 +713,16 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_occupancy<BITS, GATED, 
                 break;
             }
         }
+        static_assert(!SPLIT || NTC * 4096 <= ST, "a slab's exchange fits a stage");
+        float *const xw = reinterpret_cast<float *>(stage_base(slab)) + lane;
         if constexpr (SPLIT) {
-            if (half > 0) {   // the up waves have read the previous half
-                wait_lgkm0();
-                barrier_no_fence();
-            }
-            float *xw = xch + slab * XNT * 16 * 64 + lane;
+            wait_vm<0>();
+            barrier_no_fence();
             if (mw == 0) {
 #pragma unroll
-                for (int i = 0; i < XNT; i++) {
+                for (int i = 0; i < NTC; i++) {
 #pragma unroll
-                    for (int k = 0; k < 16; k++) xw[(i * 16 + k) * 64] = siluf_(acc0[half * XNT + i][k]);
+                    for (int k = 0; k < 16; k++) xw[(i * 16 + k) * 64] = siluf_(acc0[i][k]);
                 }
             }
             wait_lgkm0();
@@ -744,8 +730,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_occupancy<BITS, GATED, 
         }
         const int row_base = (rt0 + ti) * TR + slab * 32;
 #pragma unroll
-        for (int ii = 0; ii < XNT; ii++) {
-            const int i = half * XNT + ii;
+        for (int i = 0; i < NTC; i++) {
             const int n = 32 * i + r;
             if (n >= nvalid || (SPLIT && mw == 0)) continue;
             const int route = out_route[i];
@@ -756,7 +741,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_occupancy<BITS, GATED, 
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
                     const float g = acc0[i][4 * q + k];
-                    if constexpr (SPLIT) v[k] = xch[(slab * XNT * 16 + ii * 16 + 4 * q + k) * 64 + lane] * g;
+                    if constexpr (SPLIT) v[k] = xw[(i * 16 + 4 * q + k) * 64] * g;
                     else if constexpr (GATED) v[k] = siluf_(g) * acc1[i][4 * q + k];
                     else v[k] = g;
                 }
@@ -780,7 +765,6 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_occupancy<BITS, GATED, 
                     }
                 }
             }
-        }
         }
         zero_acc();
     }
@@ -1028,33 +1012,28 @@ bool launch_qmm(const QmmArgs &a, hipStream_t s, char *error, int capacity) {
                                        : "Chunk too large for one grouped/dense qmm launch");
         return false;
     }
-    // Route tile width: 64 routes for the gated kernels, 128 otherwise (the register-ring
-    // kernel measured faster so than with narrower tiles and deeper rings). Grouped
-    // non-gated streaming launches (K a multiple of 512) use 64: experts average a few
-    // routes, and the narrower tile lets two blocks share a CU. Exceptions by the routes
-    // per expert follow.
+    // Route tile width, by the routes an expert gets on average (8T/E):
+    // - gated, streaming: 32 routes up to 24 of them in 5 bits (77 tokens over 256 experts:
+    //   gate/up 69.7 -> 62.7 us against 64-route tiles; at 37 routes 135 -> 153 us) and up to 8
+    //   in 8 bits, where they let a second block share the CU (84.4 -> 79.4 us; at 16 routes the
+    //   popular experts' extra chunks cost as much, 143 -> 146 us), else 64, and for 5-bit
+    //   launches past 48 routes 128
+    //   (64-route tiles would give an expert of 65-127 routes a second, mostly empty chunk and
+    //   dequantize its weights twice), of which 96 are multiplied up to 64 routes: config 4
+    //   averages 64, at most ~90.
+    // - down, streaming: 32 routes up to 24 (5-bit; 77 tokens 40.9 -> 36.3 us) or 16 (8-bit;
+    //   config 3 88.7 -> 86.2 us), 96 for 5 bits past 48 (config 4 126 -> 119 us), else 64.
+    // - other K (the register-ring kernel): 64 gated, 128 otherwise.
     const bool gated = m1 != nullptr;
     const bool streaming = m0->columns % 512 == 0;
-    // 5-bit gated takes 128 route slots when experts average
-    // more than 48 routes (uniform routing over E experts: 8T/E): 64-route tiles would give
-    // an expert of 65-127 routes a second, mostly empty chunk and dequantize its weights
-    // twice (config 4: 64 routes on average, at most ~90)
-    const bool wide_gated = streaming && gated && !a.dense && qmm_wide_gated(m0, a.tokens);
-    // The grouped 5-bit down projection takes 96-route tiles (still two blocks a CU) when
-    // experts average more than 48 routes: config 4's experts (at most ~90 routes) then need
-    // one chunk each (down 126 -> 119 us; 128-route tiles, one block a CU, measured 211 ->
-    // 274 us). The 8-bit one takes 32-route tiles (three blocks a CU) when experts average
-    // at most 16 routes (config 3 down 88.7 -> 86.2 us). Others keep 64-route tiles.
-    const bool wide_down = streaming && !gated && !a.dense && m0->bits == 5 &&
-                           (size_t)a.tokens * 8 > (size_t)48 * (size_t)std::max(1, m0->experts);
-    const bool narrow_down = streaming && !gated && !a.dense && m0->bits == 8 &&
-                             (size_t)a.tokens * 8 <= (size_t)16 * (size_t)std::max(1, m0->experts);
     if (streaming && a.dense && !gated) return launch_dense_split(a, P, s, error, capacity);
-    const int nt = streaming && !a.dense && !gated ? (wide_down ? 3 : narrow_down ? 1 : 2)
-                                                   : (gated ? (wide_gated ? 4 : 2) : 4);
-    // wide 5-bit gated chunks of 96 routes when experts average at most 64 routes (the copies
-    // still fill 128 route slots; the MFMAs cover 96)
-    const int ntc = wide_gated && (size_t)a.tokens * 8 <= (size_t)64 * (size_t)std::max(1, m0->experts) ? 3 : nt;
+    const bool grouped = streaming && !a.dense;
+    const size_t routes = (size_t)a.tokens * 8, experts = (size_t)std::max(1, m0->experts);
+    const bool five = m0->bits == 5;
+    int nt = gated ? 2 : 4;
+    if (grouped && gated) nt = qmm_wide_gated(m0, a.tokens) ? 4 : routes <= (five ? 24 : 8) * experts ? 1 : 2;
+    if (grouped && !gated) nt = five && routes > 48 * experts ? 3 : routes <= (five ? 24 : 16) * experts ? 1 : 2;
+    const int ntc = nt == 4 && grouped && gated && routes <= 64 * experts ? 3 : nt;
     const int bn = 32 * ntc;
     const size_t work = qmm_max_work(m0->rows, a.tokens, a.ngroups, a.dense, bn);
     const size_t blocks = 8 * ((work + 7) / 8);
@@ -1065,17 +1044,14 @@ bool launch_qmm(const QmmArgs &a, hipStream_t s, char *error, int capacity) {
     P.max_work = (int)work;
     dim3 grid((unsigned)blocks), block(256);
     if (streaming) {
-        // row tiles per block: enough blocks to fill the GPU about twice, up to four tiles
-        // streamed back to back per block
+        // row tiles per block: two streamed back to back by a down block once the launch fills
+        // the GPU twice (four measured slower: 77 tokens 5-bit 36.3 -> 32.3 us, 200 tokens 8-bit
+        // over 128 experts 46.6 -> 42.1 us; so did single tiles, config 4 80 -> 87 us), one by a
+        // gated block, whose SwiGLU exchange takes over its stages (and finer rounds measured
+        // faster: config 4 gate/up 457 -> 380 us, config 3 166 -> 154 us)
         const size_t chunks = work / (size_t)P.row_tiles;
         const size_t per_tile = (size_t)P.row_tiles * chunks;
-        int rtb = (int)std::min<size_t>(4, std::max<size_t>(1, per_tile / 512));
-        // Gated launches (one block per CU): single row tiles. 5-bit: its work items are
-        // nearly equal, and with four tiles a block the last round of blocks ran almost empty
-        // (config 4 gate/up 457 -> 380 us). 8-bit: since the MFMAs of empty route tiles are
-        // skipped, single tiles measured faster too (config 3 gate/up 166 -> 154 us); the
-        // non-gated down projection keeps up to four (single tiles: 89 -> 101 us)
-        if (gated) rtb = 1;
+        int rtb = gated ? 1 : (int)std::min<size_t>(2, std::max<size_t>(1, per_tile / 512));
         rtb = std::min(rtb, P.row_tiles);
         P.rtb = rtb;
         P.rt_groups = (P.row_tiles + rtb - 1) / rtb;
@@ -1104,7 +1080,9 @@ bool launch_qmm(const QmmArgs &a, hipStream_t s, char *error, int capacity) {
             DIH_LAUNCH((qmm_lds_kernel<B, GT, N, 4, SP, B == 5, NC>), grid, dim3(SP ? 512 : 256), 0, s, P); \
             return hip_ok(hipGetLastError(), error, capacity, "qmm launch");        \
         }
+        DIH_QMM_LDS_CASE(8, true, 1, 1) DIH_QMM_LDS_CASE(5, true, 1, 1)
         DIH_QMM_LDS_CASE(8, true, 2, 2) DIH_QMM_LDS_CASE(8, false, 2, 2) DIH_QMM_LDS_CASE(8, false, 1, 1)
+        DIH_QMM_LDS_CASE(5, false, 1, 1)
         DIH_QMM_LDS_CASE(5, true, 2, 2) DIH_QMM_LDS_CASE(5, false, 2, 2) DIH_QMM_LDS_CASE(5, false, 3, 3)
         DIH_QMM_LDS_CASE(5, true, 4, 4) DIH_QMM_LDS_CASE(5, true, 4, 3)
 #undef DIH_QMM_LDS_CASE

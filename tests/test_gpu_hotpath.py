@@ -593,7 +593,11 @@ def _zipf_logits(rng, T, E, s=1.1):
     (100, 16, 512, 192, 5, "uniform"),  # 5-bit gate/up of 192 rows: expert codes padded to 256
     (120, 16, 512, 256, 5, "zipf"),      # 5-bit split gated, 96-route chunks, popular experts split
     (100, 16, 512, 512, 5, "zipf"),      # 5-bit down in 96-route tiles (experts average 50 routes)
-    (200, 16, 512, 256, 5, "uniform")])  # 5-bit split gated in 128-route chunks (experts average 100)
+    (200, 16, 512, 256, 5, "uniform"),   # 5-bit split gated in 128-route chunks (experts average 100)
+    (48, 16, 1024, 512, 5, "zipf"), (16, 16, 1024, 512, 8, "zipf"),   # 24 and 8 routes an expert: 32-route
+    (49, 16, 1024, 512, 5, "zipf"), (17, 16, 1024, 512, 8, "zipf"),   # gated tiles; just past: 64
+    (40, 64, 512, 512, 8, "zipf"),       # 32-route gated chunks, popular experts in two
+    (32, 16, 512, 1024, 8, "uniform"), (3, 64, 512, 512, 5, "zipf")])  # 16 routes: 8-bit down in 32-route tiles
 def test_moe_prefill_matches_oracle(device, T, E, H, I, bits, routing):
     rng = np.random.default_rng(T * 7 + E)
     L = _moe_layer(rng, E, H, I, bits, router=False)
