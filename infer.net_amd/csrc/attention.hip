@@ -14,7 +14,8 @@
 //                 query row (lane & 31) and 16 of the tile's keys, so the row maximum and
 //                 sum need one exchange with lane ^ 32 and the probabilities are already
 //                 the B operand of the next product;
-//   O^T += V^T P^T  16 MFMAs (A = the tile's values transposed into LDS, B = the bf16
+//   O^T += V^T P^T  16 MFMAs (A = the tile's values, transposed on the way into LDS by the
+//                 four-wave block, read transposed by the eight-wave one, B = the bf16
 //                 probabilities), again one row per lane: the rescale by exp(m_old - m_new)
 //                 and the final 1/sum are lane-local.
 // Probabilities are exp(s - m) against the running maximum including the current tile,
@@ -81,13 +82,15 @@ DIH_DEV void store_out4(const AttnParams &P, int tok, int head, int d0, const fl
     }
 }
 
-// Keys reach LDS by direct global->LDS copies (no registers): key row kl (512 B) holds its
-// 16-byte piece c at slot c ^ (kl & 15), which makes the MFMA operand reads (16 lanes = 16
-// keys, one piece each) conflict-free. Of a block of NW waves, wave w copies rows
-// (32/NW)w .. (32/NW)(w+1)-1, two rows per instruction. Key indices past the partition end
-// are clamped to its last key (finite data; those keys are masked).
+// Keys and values reach LDS by direct global->LDS copies (no registers), untransposed: row kl
+// (512 B) holds its 16-byte piece c at slot c ^ swizzle(kl). Keys: kl & 15, which makes the
+// MFMA operand reads (16 lanes = 16 keys, one piece each) conflict-free. Values read through
+// transposing reads (TR): 4 * (kl & 3), which puts the four keys of such a read on four
+// bank groups. Of a block of NW waves, wave w copies rows (32/NW)w .. (32/NW)(w+1)-1, two rows
+// per instruction. Key indices past the partition end are clamped to its last key (finite
+// data; those keys are masked).
 template <int NW>
-DIH_DEV void issue_keys(const uint16_t *kbase, uint16_t *ksbuf, int kb, int kend, int wave, int lane) {
+DIH_DEV void issue_rows(const uint16_t *base, uint16_t *buf, int kb, int kend, int wave, int lane) {
     constexpr int RPW = kKeys / NW;   // rows per wave, two per copy instruction
 #pragma unroll
     for (int i = 0; i < RPW / 2; i++) {
@@ -96,16 +99,8 @@ DIH_DEV void issue_keys(const uint16_t *kbase, uint16_t *ksbuf, int kb, int kend
         const uint32_t key = (uint32_t)min(kb + kl, kend - 1);
         // 32-bit element offset from the wave-uniform base (the cache is below 2^31 elements)
         const uint32_t off = key * (uint32_t)(kKvHeads * kDim) + 8u * (uint32_t)c;
-        to_lds<16>(kbase + off, ksbuf + (RPW * wave + 2 * i) * kDim);
+        to_lds<16>(base + off, buf + (RPW * wave + 2 * i) * kDim);
     }
-}
-
-// Values reach LDS the same way, untransposed (raw rows of 512 B, piece c at slot
-// c ^ (kl & 15)), into one buffer that is consumed by the transpose below before the next
-// tile's copies are issued.
-template <int NW>
-DIH_DEV void issue_values(const uint16_t *vbase, uint16_t *vraw, int kb, int kend, int wave, int lane) {
-    issue_keys<NW>(vbase, vraw, kb, kend, wave, lane);
 }
 
 DIH_DEV void store_vt_pair(uint16_t *vt, int d, int vq, uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3) {
@@ -133,28 +128,6 @@ DIH_DEV void transpose_values(const uint16_t *vraw, uint16_t *vt, int vq, int vc
     store_vt_pair(vt, d + 2, vq, v[0].y, v[1].y, v[2].y, v[3].y);
     store_vt_pair(vt, d + 4, vq, v[0].z, v[1].z, v[2].z, v[3].z);
     store_vt_pair(vt, d + 6, vq, v[0].w, v[1].w, v[2].w, v[3].w);
-}
-
-// The same for 512 threads: thread t reads 4 dims (4*(t/8)..+3) of keys 4*(t%8)..+3.
-DIH_DEV void transpose_values8(const uint16_t *vraw, uint16_t *vt, int t) {
-    const int vq = t & 7, vd = t >> 3;
-    uint2 v[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int kl = 4 * vq + i;
-        v[i] = *reinterpret_cast<const uint2 *>(vraw + kl * kDim + 8 * ((vd >> 1) ^ (kl & 15)) + 4 * (vd & 1));
-    }
-    // word x of each key holds dims 4vd (low half), 4vd+1; word y dims 4vd+2, 4vd+3
-    const uint32_t lo[4] = {v[0].x, v[1].x, v[2].x, v[3].x}, hi[4] = {v[0].y, v[1].y, v[2].y, v[3].y};
-    uint16_t *row = vt + 4 * vd * kVtStride + 4 * vq;
-    *reinterpret_cast<uint2 *>(row) = make_uint2(__builtin_amdgcn_perm(lo[1], lo[0], 0x05040100u),
-                                                 __builtin_amdgcn_perm(lo[3], lo[2], 0x05040100u));
-    *reinterpret_cast<uint2 *>(row + kVtStride) = make_uint2(__builtin_amdgcn_perm(lo[1], lo[0], 0x07060302u),
-                                                             __builtin_amdgcn_perm(lo[3], lo[2], 0x07060302u));
-    *reinterpret_cast<uint2 *>(row + 2 * kVtStride) = make_uint2(__builtin_amdgcn_perm(hi[1], hi[0], 0x05040100u),
-                                                                 __builtin_amdgcn_perm(hi[3], hi[2], 0x05040100u));
-    *reinterpret_cast<uint2 *>(row + 3 * kVtStride) = make_uint2(__builtin_amdgcn_perm(hi[1], hi[0], 0x07060302u),
-                                                                 __builtin_amdgcn_perm(hi[3], hi[2], 0x07060302u));
 }
 
 // ---- the parts of a wave's work shared by both block shapes. A wave owns 32 rows: 4
@@ -201,15 +174,8 @@ DIH_DEV uint32_t scale_bf16x2(uint32_t w, float f) {
     return pack_bf16x2(__uint_as_float(w << 16) * f, __uint_as_float(w & 0xffff0000u) * f);
 }
 
-// One 32-key tile (keys kb.., rows from ksb, values transposed in vtb) for the wave's rows.
-// `full`: every row of the wave sees the whole tile (no mask needed). RESTARTS: the block's
-// keys span more than one rounding partition; `restart`: this tile starts one (and is not
-// the block's first tile).
-template <bool RESTARTS>
-DIH_DEV void attend_tile(const uint16_t *ksb, const uint16_t *vtb, const dih_bf16x8 (&qreg)[16],
-                         dih_f32x16 (&acc)[8], RowState &st, int kb, int kend, bool full, bool restart,
-                         int my_last, int r, int h) {    // ---- S^T = K Q^T: s[k] is key kb + 8(k/4) + 4h + k%4 of row r
-    dih_f32x16 s;
+// S^T = K Q^T of one 32-key tile (rows from ksb): s[k] is key kb + 8(k/4) + 4h + k%4 of row r.
+DIH_DEV void qk_tile(const uint16_t *ksb, const dih_bf16x8 (&qreg)[16], dih_f32x16 &s, int r, int h) {
 #pragma unroll
     for (int k = 0; k < 16; k++) s[k] = 0.f;
 #pragma unroll
@@ -217,8 +183,25 @@ DIH_DEV void attend_tile(const uint16_t *ksb, const uint16_t *vtb, const dih_bf1
         const dih_bf16x8 a = *reinterpret_cast<const dih_bf16x8 *>(ksb + r * kDim + 8 * ((2 * st + h) ^ (r & 15)));
         s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qreg[st], s, 0, 0, 0);
     }
-    // ---- online softmax for row r. Scores stay raw here; the log2 scale enters the
-    // exponent's FMA.
+}
+
+// v combined with the value of lane ^ 32 (the other half's keys of the same row), without LDS.
+template <typename Op>
+DIH_DEV float half_reduce(float v, Op op) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return op(__builtin_bit_cast(float, (uint32_t)p[0]), __builtin_bit_cast(float, (uint32_t)p[1]));
+}
+
+// Online softmax of the tile's scores for row r: the probabilities as bf16 pairs (pw: the B
+// operands of the next product) and the row's state. Returns the factor that takes the
+// row's accumulators to its new scale.
+// Scores stay raw; the log2 scale enters the exponent's FMA. `full`: every row of the wave
+// sees the whole tile (no mask needed). RESTARTS: the block's keys span more than one
+// rounding partition; `restart`: this tile starts one (and is not the block's first tile).
+template <bool RESTARTS>
+DIH_DEV float softmax_tile(dih_f32x16 &s, uint32_t (&pw)[8], RowState &st, int kb, int kend, bool full, bool restart,
+                           int my_last, int h) {
     float mx = -INFINITY;
     if (full) {
 #pragma unroll
@@ -231,7 +214,7 @@ DIH_DEV void attend_tile(const uint16_t *ksb, const uint16_t *vtb, const dih_bf1
             mx = fmaxf(mx, s[k]);
         }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = half_reduce(mx, OpMax());
     const float tmax = mx * kLog2eOver16;
     float r_new, alpha, f = 1.f;
     if constexpr (RESTARTS) {
@@ -251,7 +234,6 @@ DIH_DEV void attend_tile(const uint16_t *ksb, const uint16_t *vtb, const dih_bf1
     st.m = r_new;
     const float m_use = r_new == -INFINITY ? 0.f : r_new;   // all keys masked: p = 0
     float psum = 0.f;
-    uint32_t pw[8];
 #pragma unroll
     for (int k = 0; k < 16; k += 2) {
         const float p0 = __builtin_amdgcn_exp2f(fmaf(s[k], kLog2eOver16, -m_use));
@@ -259,23 +241,34 @@ DIH_DEV void attend_tile(const uint16_t *ksb, const uint16_t *vtb, const dih_bf1
         psum += p0 + p1;
         pw[k >> 1] = pack_bf16x2(p0, p1);
     }
-    psum += __shfl_xor(psum, 32, 64);
-    st.sum = st.sum * alpha + psum * f;
+    st.sum = st.sum * alpha + half_reduce(psum, OpAdd()) * f;
     // probabilities of a partition far below the scale: rounded above, then scaled exactly
     if (RESTARTS && __ballot(f != 1.f)) {
 #pragma unroll
         for (int i = 0; i < 8; i++) pw[i] = scale_bf16x2(pw[i], f);
     }
-    // rescale only when some row's scale moved (alpha == 1 exactly otherwise)
-    if (__ballot(alpha != 1.f)) {
+    return alpha;
+}
+
+// The accumulators in their rows' new scale; nothing to do when no row's moved (alpha == 1
+// exactly).
+DIH_DEV void rescale(dih_f32x16 (&acc)[8], float alpha) {
+    if (!__ballot(alpha != 1.f)) return;
 #pragma unroll
-        for (int dt = 0; dt < 8; dt++)
+    for (int dt = 0; dt < 8; dt++)
 #pragma unroll
-            for (int k = 0; k < 16; k++) acc[dt][k] *= alpha;
-    }
+        for (int k = 0; k < 16; k++) acc[dt][k] *= alpha;
+}
+
+DIH_DEV dih_bf16x8 pv_operand(uint2 lo, uint2 hi) {
+    return __builtin_bit_cast(dih_bf16x8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+}
+
+// O^T += V^T P^T from values transposed in vtb: acc[dt][k] is dim 32dt + 8(k/4) + 4h + k%4 of
+// row r.
+DIH_DEV void pv_tile(const uint16_t *vtb, const uint32_t (&pw)[8], dih_f32x16 (&acc)[8], int r, int h) {
     const dih_bf16x8 pb0 = __builtin_bit_cast(dih_bf16x8, make_uint4(pw[0], pw[1], pw[2], pw[3]));
     const dih_bf16x8 pb1 = __builtin_bit_cast(dih_bf16x8, make_uint4(pw[4], pw[5], pw[6], pw[7]));
-    // ---- O^T = O^T * alpha + V^T P^T: acc[dt][k] is dim 32dt + 8(k/4) + 4h + k%4 of row r
 #pragma unroll
     for (int dt = 0; dt < 8; dt++) {
         const uint16_t *vrow = vtb + (32 * dt + r) * kVtStride + 4 * h;
@@ -283,10 +276,8 @@ DIH_DEV void attend_tile(const uint16_t *ksb, const uint16_t *vtb, const dih_bf1
         const uint2 a1 = *reinterpret_cast<const uint2 *>(vrow + 8);
         const uint2 a2 = *reinterpret_cast<const uint2 *>(vrow + 16);
         const uint2 a3 = *reinterpret_cast<const uint2 *>(vrow + 24);
-        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            __builtin_bit_cast(dih_bf16x8, make_uint4(a0.x, a0.y, a1.x, a1.y)), pb0, acc[dt], 0, 0, 0);
-        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            __builtin_bit_cast(dih_bf16x8, make_uint4(a2.x, a2.y, a3.x, a3.y)), pb1, acc[dt], 0, 0, 0);
+        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pv_operand(a0, a1), pb0, acc[dt], 0, 0, 0);
+        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pv_operand(a2, a3), pb1, acc[dt], 0, 0, 0);
     }
 }
 
@@ -356,8 +347,8 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnParams P) {
 #pragma unroll
         for (int k = 0; k < 16; k++) acc[i][k] = 0.f;
 
-    issue_keys<4>(kbase, ks[0], kstart, kend, wave, lane);
-    issue_values<4>(vbase, vraw, kstart, kend, wave, lane);
+    issue_rows<4>(kbase, ks[0], kstart, kend, wave, lane);
+    issue_rows<4>(vbase, vraw, kstart, kend, wave, lane);
     int buf = 0;
     for (int kb = kstart; kb < kend; kb += kKeys, buf ^= 1) {
         wait_vm<0>();             // this thread's copies have landed
@@ -365,32 +356,109 @@ __global__ __launch_bounds__(256, 2) void attn_kernel(AttnParams P) {
         transpose_values(vraw, vt, vq, vc);
         __syncthreads();          // vt complete, vraw consumed
         if (kb + kKeys < kend) {
-            issue_keys<4>(kbase, ks[buf ^ 1], kb + kKeys, kend, wave, lane);
-            issue_values<4>(vbase, vraw, kb + kKeys, kend, wave, lane);
+            issue_rows<4>(kbase, ks[buf ^ 1], kb + kKeys, kend, wave, lane);
+            issue_rows<4>(vbase, vraw, kb + kKeys, kend, wave, lane);
         }
         if (!wave_ok || kb > wave_last) continue;
         const bool full = kb + kKeys - 1 <= P.position + wtok0 && kb + kKeys <= kend;
-        attend_tile<RESTARTS>(ks[buf], vt, qreg, acc, st, kb, kend, full,
-                              RESTARTS && kb != kstart && kb % P.round == 0, my_last, r, h);
+        dih_f32x16 s;
+        uint32_t pw[8];
+        qk_tile(ks[buf], qreg, s, r, h);
+        rescale(acc, softmax_tile<RESTARTS>(s, pw, st, kb, kend, full, RESTARTS && kb != kstart && kb % P.round == 0,
+                                            my_last, h));
+        pv_tile(vt, pw, acc, r, h);
     }
     if (!row_ok) return;
     finish_rows(P, acc, st, my_tok, head, part, h);
 }
 
-// ---- eight-wave form: 32 query tokens (256 rows) per block share each key/value tile.
-// Keys are triple-buffered and values double-buffered (raw copies and transposed), so one
-// barrier per tile suffices and every tile's copies are issued two tiles ahead:
-//   top of tile j: tile j's keys and transposed values are in LDS, tile j+1's copies landed
-//   issue tile j+2's copies (into the buffers tile j-1 used), compute tile j, transpose
-//   tile j+1's values, wait for this thread's copies, barrier.
+// The multiplying half of an eight-wave block's step: O^T += V^T P^T of one tile (values at LDS
+// byte address vs), then S^T = K Q^T of the next (keys at ks). Keys: row n at 512 n, 16-byte
+// piece c at slot c ^ (n & 15). Values: row n at 512 n, piece c at slot c ^ 4 (n & 3), through
+// transposing reads: in each group of 16 lanes, lane 4e + c addresses dims 4c..4c+3 of key e of
+// four, and lane i receives dim i of the four keys; the swizzle puts the four keys on four
+// bank groups. `copy(i)`, i = 0..3, issues a copy of a later tile.
+template <typename F>
+DIH_DEV void multiply_tile(uint32_t vs, uint32_t ks, const uint32_t (&pw)[8], const dih_bf16x8 (&qreg)[16],
+                           dih_f32x16 (&acc)[8], dih_f32x16 &s, int lane, F copy) {
+    typedef short v4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) v4 lds_v4;
+    typedef __attribute__((address_space(3))) const dih_bf16x8 lds_bf16x8;
+    const dih_bf16x8 pb0 = __builtin_bit_cast(dih_bf16x8, make_uint4(pw[0], pw[1], pw[2], pw[3]));
+    const dih_bf16x8 pb1 = __builtin_bit_cast(dih_bf16x8, make_uint4(pw[4], pw[5], pw[6], pw[7]));
+    const uint32_t h = (uint32_t)lane >> 5, r = (uint32_t)lane & 31, e = ((uint32_t)lane >> 2) & 3;
+    // keys 4h + e (and + 8, + 16, + 24), dims 32 dt + 16 ((lane >> 4) & 1) + 4 (lane & 3) ..
+    const uint32_t va = vs + (4 * h + e) * 512 + (e << 6) + ((uint32_t)(lane & 16) << 1) + ((uint32_t)(lane & 3) << 3);
+    const uint32_t ka = ks + r * 512 + ((h ^ (r & 15)) << 4);
+    auto vread = [&](int dt, int k8) {
+        const uint32_t at = (va ^ (uint32_t)((dt & 3) << 6)) + (uint32_t)((dt & 4) * 64 + k8 * 4096);
+        return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4 *)(uintptr_t)at));
+    };
+    auto kread = [&](int st) {
+        return *(lds_bf16x8 *)(uintptr_t)((ka ^ (uint32_t)((st & 7) << 5)) + (uint32_t)((st & 8) << 5));
+    };
+    // The compiler may not move work between the stages below (it would wait on each read just
+    // after issuing it). V^T P^T: a stage a dim tile, its operands read kV stages before.
+    constexpr int kV = 2, kK = 4;
+    uint2 a[kV + 1][4];
+    dih_bf16x8 kk[kK + 2];
+#pragma unroll
+    for (int dt = 0; dt < kV; dt++)
+#pragma unroll
+        for (int k8 = 0; k8 < 4; k8++) a[dt][k8] = vread(dt, k8);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int dt = 0; dt < 8; dt++) {
+        const int b = dt % (kV + 1);
+        if (dt + kV < 8) {
+#pragma unroll
+            for (int k8 = 0; k8 < 4; k8++) a[(dt + kV) % (kV + 1)][k8] = vread(dt + kV, k8);
+        } else {   // the first key pieces
+            kk[2 * (dt + kV - 8)] = kread(2 * (dt + kV - 8));
+            kk[2 * (dt + kV - 8) + 1] = kread(2 * (dt + kV - 8) + 1);
+        }
+        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pv_operand(a[b][0], a[b][1]), pb0, acc[dt], 0, 0, 0);
+        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pv_operand(a[b][2], a[b][3]), pb1, acc[dt], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // K Q^T: a stage two key pieces, read kK pieces before
+    const dih_f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int st = 0; st < 16; st += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            if (st + u + kK < 16) kk[(st + u + kK) % (kK + 2)] = kread(st + u + kK);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kk[(st + u) % (kK + 2)], qreg[st + u], st + u ? s : zero, 0, 0, 0);
+        if (st & 2) copy(st >> 2);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// ---- eight-wave form: 32 query tokens (256 rows) per block share each key/value tile. Waves
+// w and w + 4 share a SIMD, and the two groups run the same loop half a step apart: while one
+// group's wave multiplies (V^T P^T of tile j, then K Q^T of tile j + 1), the other's computes a
+// softmax, with a barrier at every change. Bound by the two halves, 1,500-1,800 cycles each of
+// a tile's 4,150: the softmax by its VALU work (121 instructions, 16 exponentials among them,
+// and 128 multiplies where a row's scale moves), the products by MFMAs (1,024) and the latency
+// of their operand reads. In lockstep, with one accumulator set and its spills, MFMAs, LDS
+// reads, softmax and the values' transposition took turns: 7,500 cycles a tile. The last
+// 2048-token chunk of a 32K prompt 1,610 -> 1,099 us, 2048 tokens from position 0 119 -> 98
+// us, 837 tokens at position 18,686 671 -> 436 us. Spreading the rescale over the MFMAs, two
+// score chains and alternating the products were each no faster (more registers, so shorter
+// operand read-ahead).
+// Keys and values are triple-buffered raw rows: step j reads values j and keys j + 1, and
+// requests values j + 2 and keys j + 3 into the slots that step j - 1 read, so a copy has more
+// than a step to land. Tiles past the last are requested clamped to the partition's last key
+// (their products are masked or never read), which keeps the waits' counts constant.
 template <bool RESTARTS>
 __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
     __shared__ __align__(16) uint16_t ks[3][kKeys * kDim];
-    __shared__ __align__(16) uint16_t vraw[2][kKeys * kDim];
-    __shared__ __align__(16) uint16_t vt[2][kDim * kVtStride];
-    lds_escape(ks, vraw, vt);
+    __shared__ __align__(16) uint16_t vs[3][kKeys * kDim];
+    lds_escape(ks, vs);
 
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63, r = lane & 31, h = lane >> 5;
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, r = lane & 31, h = lane >> 5;
     // work item: as attn_kernel, with 32-token tiles
     const int b = blockIdx.x, x = b & 7, kh = x >> 2;
     const int idx = (x & 3) + 4 * (b >> 3);
@@ -403,14 +471,8 @@ __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
     if (kstart >= kend) return;
 
     const int wtok0 = tok0 + 4 * wave;
-    const bool wave_ok = wtok0 < P.tokens;
-    const int wave_last = P.position + min(wtok0 + 3, P.tokens - 1);
-    const int my_tok = wtok0 + (r >> 3), head = kh * kGroup + (r & 7);
-    const bool row_ok = my_tok < P.tokens;
-    const int my_last = row_ok ? P.position + my_tok : -1;
-
     dih_bf16x8 qreg[16];
-    load_queries(qreg, P, my_tok, row_ok, head, h);
+    load_queries(qreg, P, wtok0 + (r >> 3), wtok0 + (r >> 3) < P.tokens, kh * kGroup + (r & 7), h);
     RowState st;
     dih_f32x16 acc[8];
 #pragma unroll
@@ -420,42 +482,85 @@ __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
 
     const uint16_t *kbase = P.keys + kh * kDim, *vbase = P.values + kh * kDim;
     const int ntile = (kend - kstart + kKeys - 1) / kKeys;
-    issue_keys<8>(kbase, ks[0], kstart, kend, wave, lane);
-    issue_values<8>(vbase, vraw[0], kstart, kend, wave, lane);
-    if (ntile > 1) {
-        issue_keys<8>(kbase, ks[1], kstart + kKeys, kend, wave, lane);
-        issue_values<8>(vbase, vraw[1], kstart + kKeys, kend, wave, lane);
-        wait_vm<4>();         // tile 0's four copies of this thread (tile 1's may stay in flight)
-    } else {
-        wait_vm<0>();
-    }
-    barrier_no_fence();
-    transpose_values8(vraw[0], vt[0], t);
-    wait_vm<0>();
-    wait_lgkm0();
-    barrier_no_fence();
-
-    int k3 = 0;   // j % 3
-    for (int j = 0; j < ntile; j++) {
+    dih_f32x16 s;
+    uint32_t pw[8];
+    // Copy i of a tile's keys (or values) by this wave: rows 4 * wave + 2i and the next one, from
+    // the block's first key on, a lane 16 bytes; rows past the partition's end repeat its last
+    // key (finite data; those keys are masked). Untracked by the compiler (as copy16_to_lds,
+    // without a memory clobber: nothing reads the slot before the barrier the copies are waited
+    // for at): it would make the first operand read of a step wait for the copies just issued.
+    const uint16_t *const kfirst = kbase + (size_t)kstart * (kKvHeads * kDim);
+    const uint16_t *const vfirst = vbase + (size_t)kstart * (kKvHeads * kDim);
+    const uint32_t ks_lds = (uint32_t)(uintptr_t)&ks[0][0], vs_lds = (uint32_t)(uintptr_t)&vs[0][0];
+    constexpr uint32_t kSlot = kKeys * kDim * 2;
+    auto copy = [&](const uint16_t *base, uint32_t slot, bool keys, int j, int i, int l) {
+        const int kl = 4 * wave + 2 * i + (l >> 5);
+        const uint32_t c = (uint32_t)((l & 31) ^ (keys ? kl & 15 : 4 * (kl & 3)));
+        const uint32_t row = (uint32_t)min(j * kKeys + kl, kend - kstart - 1);
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(row << 10 | c << 4),
+                     "s"(base), "s"(slot + (uint32_t)(4 * wave + 2 * i) * (kDim * 2))
+                     : "m0");
+    };
+    static_assert(kKvHeads * kDim * 2 == 1 << 10, "bytes of a cache row");
+    auto keys = [&](int j, int slot) {
+        for (int i = 0; i < 2; i++) copy(kfirst, ks_lds + (uint32_t)slot * kSlot, true, j, i, lane);
+    };
+    auto values = [&](int j, int slot) {
+        for (int i = 0; i < 2; i++) copy(vfirst, vs_lds + (uint32_t)slot * kSlot, false, j, i, lane);
+    };
+    // What depends on the lane is formed anew in every phase, from a lane index the compiler
+    // cannot see through: held across the loop it would spill, and a spill's reload waits for
+    // every copy in flight.
+    auto fresh = [&]() {
+        int l = lane;
+        asm volatile("" : "+v"(l));
+        return l;
+    };
+    // (every wave takes part in every tile: rows that see none of its keys have masked scores,
+    // which leave their state and accumulators as they are)
+    auto soften = [&](int j) {
         const int kb = kstart + j * kKeys;
-        if (j + 2 < ntile) {
-            const int k3n = k3 == 0 ? 2 : k3 - 1;   // (j + 2) % 3
-            issue_keys<8>(kbase, ks[k3n], kb + 2 * kKeys, kend, wave, lane);
-            issue_values<8>(vbase, vraw[j & 1], kb + 2 * kKeys, kend, wave, lane);
-        }
-        if (wave_ok && kb <= wave_last) {
-            const bool full = kb + kKeys - 1 <= P.position + wtok0 && kb + kKeys <= kend;
-            attend_tile<RESTARTS>(ks[k3], vt[j & 1], qreg, acc, st, kb, kend, full,
-                                  RESTARTS && kb != kstart && kb % P.round == 0, my_last, r, h);
-        }
-        if (j + 1 < ntile) transpose_values8(vraw[(j + 1) & 1], vt[(j + 1) & 1], t);
-        wait_vm<0>();
-        wait_lgkm0();
+        const bool full = kb + kKeys - 1 <= P.position + wtok0 && kb + kKeys <= kend;
+        const int l = fresh(), my_tok = wtok0 + ((l & 31) >> 3);
+        rescale(acc, softmax_tile<RESTARTS>(s, pw, st, kb, kend, full, RESTARTS && j != 0 && kb % P.round == 0,
+                                            my_tok < P.tokens ? P.position + my_tok : -1, l >> 5));
+    };
+    auto flip = [&]() {   // every wave's LDS reads of the phase are done
+        __builtin_amdgcn_sched_barrier(0);
         barrier_no_fence();
-        k3 = k3 == 2 ? 0 : k3 + 1;
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    keys(0, 0);
+    keys(1, 1);
+    values(0, 0);
+    keys(2, 2);
+    values(1, 1);
+    wait_vm<8>();    // (two copies a call: keys 0 have landed)
+    flip();
+    qk_tile(ks[0], qreg, s, r, h);
+    wait_vm<4>();    // keys 1 and values 0
+    flip();
+    int s0 = 0, s1 = 1, s2 = 2;   // slots of tiles j, j + 1, j + 2
+    if (wave >= 4) flip();        // the second group runs one phase behind
+    for (int j = 0; j < ntile; j++) {
+        soften(j);
+        flip();
+        const int l = fresh();
+        multiply_tile(vs_lds + (uint32_t)s0 * kSlot, ks_lds + (uint32_t)s1 * kSlot, pw, qreg, acc, s, l, [&](int i) {
+            if (i < 2) copy(vfirst, vs_lds + (uint32_t)s2 * kSlot, false, j + 2, i, l);
+            else copy(kfirst, ks_lds + (uint32_t)s0 * kSlot, true, j + 3, i - 2, l);
+        });
+        wait_vm<4>();   // the next step's keys and values
+        flip();
+        const int o = s0;
+        s0 = s1;
+        s1 = s2;
+        s2 = o;
     }
-    if (!row_ok) return;
-    finish_rows(P, acc, st, my_tok, head, part, h);
+    if (wave < 4) flip();
+    wait_vm<0>();   // no copy may still be writing this block's LDS when the block exits
+    const int l = fresh(), my_tok = wtok0 + ((l & 31) >> 3);
+    if (my_tok < P.tokens) finish_rows(P, acc, st, my_tok, kh * kGroup + (l & 7), part, l >> 5);
 }
 
 // One wave per (token, head), four dims per lane: merge the partitions that hold keys of

@@ -280,6 +280,17 @@ DIH_DEV void to_lds(const void *src, void *lds_wave_base) {
         __builtin_amdgcn_global_load_lds((gbl_void_t *)src, (lds_void_t *)lds_wave_base, 4, 0, 0);
 }
 
+// Direct copy global -> LDS of 16 bytes a lane: lane i's bytes from base + off land at LDS byte
+// lds + 16 i; M0 holds the wave's LDS destination. Issued as inline asm,
+// so that the compiler does not track these LDS writes: it would otherwise make every LDS
+// read wait for all copies in flight, since it cannot tell the stages apart. The kernels
+// order the copies themselves (vmcnt waits on their own copies, then a barrier, before a
+// stage is read).
+DIH_DEV void copy16_to_lds(const void *base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+                 : "memory", "m0");
+}
+
 // s_waitcnt vmcnt(N) leaving the other counters alone (gfx9 encoding)
 template <int N>
 DIH_DEV void wait_vm() {

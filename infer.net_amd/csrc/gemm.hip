@@ -155,17 +155,6 @@ DIH_DEV void staged_store(const dih_f32x16 (&acc)[WTM][WTN], unsigned char *buf,
     }
 }
 
-// Direct copies global -> LDS of 16 (or 4) bytes a lane: lane i's bytes from base + off land
-// at LDS byte lds + 16 i (or 4 i); M0 holds the wave's LDS destination. Issued as inline asm,
-// so that the compiler does not track these LDS writes: it would otherwise make every LDS
-// read wait for all copies in flight, since it cannot tell the stages apart. The kernels
-// order the copies themselves (vmcnt waits on their own copies, then a barrier, before a
-// stage is read).
-DIH_DEV void copy16_to_lds(const void *base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
-                 : "memory", "m0");
-}
-
 struct GemmParams {
     const uint16_t *w;          // [R][C] bf16 weights
     const uint16_t *x;          // [T][C] bf16

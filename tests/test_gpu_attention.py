@@ -180,6 +180,26 @@ def test_attention_bf16_operands(device, inputs):
     assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + ABS_TOL)
 
 
+@pytest.mark.parametrize("position,count", [(0, 33), (1, 36), (30, 63), (33, 94), (63, 97), (94, 35), (160, 61)])
+def test_attention_eight_wave_edges(device, inputs, position, count):
+    """Chunks of 32-token blocks whose last block is ragged by a token, a wave (4 tokens) or most of
+    itself, over one to nine key tiles (fewer, as many and more than the three tiles in LDS), the last
+    tile full or partial; rows past the chunk hold NaN."""
+    I = inputs
+    end = position + count
+    dk, dv = I.dk.clone(), I.dv.clone()
+    dk[end:] = 0x7fc0
+    dv[end:] = 0x7fc0
+    out = torch.full((256, 4096), float("nan"), device="cuda")
+    dh.attention(device, I.dq, dk, dv, I.draw, out, position, count)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    want = orc.attention_f64(I.q[:count], I.k, I.v, I.raw[:count], position,
+                             partition=dh.attention_partition(position, count))
+    _check(got[:count], want)
+    assert np.all(np.isnan(got[count:]))
+
+
 @pytest.mark.parametrize("position", [0, 31, 32, 96, 127, 128, 129, 255, 1000, 8191])
 def test_attention_decode_positions(device, inputs, position):
     """One decode token (the decode kernels: 128-key blocks of four 32-key tiles, after the
