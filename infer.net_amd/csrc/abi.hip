@@ -1240,7 +1240,8 @@ __attribute__((visibility("default"))) int dih_delta_rule(void *ctx, float *stat
         a.qp = static_cast<float *>(ctx_scratch(c, S_DQ, tiles * 32 * 128 * 4, error, capacity));
         a.cu = static_cast<float *>(ctx_scratch(c, S_DCU, tiles * 32 * 128 * 4, error, capacity));
         a.factors = static_cast<float *>(ctx_scratch(c, S_DF, tiles * 32 * 2 * 4, error, capacity));
-        if (!a.w || !a.u || !a.qp || !a.cu || !a.factors) return -1;
+        a.kf = static_cast<float *>(ctx_scratch(c, S_DK, tiles * 16 * 128 * 4, error, capacity));
+        if (!a.w || !a.u || !a.qp || !a.cu || !a.factors || !a.kf) return -1;
     }
     hipStream_t s = pick(c, stream);
     ProfScope prof_scope(c);

@@ -34,6 +34,7 @@ struct DeltaParams {
     const float *conv, *decay, *beta, *raw;
     float *state, *history, *out;
     float *w, *u, *qp, *cu, *factors;   // chunkwise scratch, indexed by tile = block * 32 + head
+    float *kf;                          // keys, indexed by block * 16 + key head
     int tokens, nblocks;
 };
 
@@ -181,7 +182,11 @@ __global__ __launch_bounds__(256) void delta_seq_kernel(DeltaParams P) {
     if (blockIdx.x < kRowLen / 256) roll_history(P, blockIdx.x * 256 + tid);
 }
 
-// ---- chunkwise prepare: one block per (head, 32-token block), 4 waves.
+// ---- chunkwise prepare: one block per (head, 32-token block), 4 waves. Its serial phases
+// (loads, products, inverse) leave the matrix pipes idle in turn, so what counts is how many
+// blocks share a CU: the values, read by one wave only, stay in registers, and 53 KB of LDS
+// let three blocks run where 70 KB let two. 2,048 tokens: 76-79 -> 59-61 us, 62-66 with the
+// operands written in apply's order (which that kernel wins back twice over).
 constexpr int kApplyRows = 16;   // value rows per apply block
 constexpr int kPad4 = kDim + 4;   // f32 row stride of [32][128] tiles: 16-byte rows, conflict-free 128-bit reads
 constexpr int kSq4 = kBlk + 4;    // f32 row stride of [32][32] and [128][32] tiles, same property
@@ -197,8 +202,8 @@ DIH_DEV void load_rows4(float *dst, const float *src_row0, int tid, int valid, i
     }
 }
 
-__global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaParams P) {
-    __shared__ __align__(16) float ks[kBlk * kPad4], qs[kBlk * kPad4], vs[kBlk * kPad4];
+__global__ __launch_bounds__(256, 3) void delta_prepare_kernel(DeltaParams P) {
+    __shared__ __align__(16) float ks[kBlk * kPad4], qs[kBlk * kPad4];
     // K K^T and Q K^T, each as two partial sums over the halves of the key dims; then C over
     // the first Q K^T half, L over the first K K^T half, T over the second K K^T half
     __shared__ __align__(16) float kkp[2][kBlk * kSq4], qkp[2][kBlk * kSq4];
@@ -212,7 +217,14 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaParams P) {
 
     load_rows4(ks, rows, tid, valid, kK + kh * kDim);
     load_rows4(qs, rows, tid, valid, kQ + kh * kDim);
-    load_rows4(vs, rows, tid, valid, kV + head * kDim);
+    // the values this thread multiplies (tokens 16h..16h+15 of dim 32 wave + r) stay in registers
+    float vj[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const int t = 16 * h + i;
+        const float v = rows[(size_t)min(t, valid - 1) * kRowLen + kV + head * kDim + 32 * wave + r];
+        vj[i] = t < valid ? v : 0.f;
+    }
     if (tid < kBlk) {
         a[tid] = tid < valid ? P.decay[(base + tid) * kVHeads + head] : 1.f;
         b[tid] = tid < valid ? P.beta[(base + tid) * kVHeads + head] : 0.f;
@@ -341,7 +353,7 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaParams P) {
             for (int e = 0; e < 4; e++) {
                 const int j = 16 * h + 4 * m + e;
                 wa = mfma_f32(t4[e], bg[j] * ks[j * kPad4 + dcol], wa);
-                ua = mfma_f32(t4[e], b[j] * vs[j * kPad4 + dcol], ua);
+                ua = mfma_f32(t4[e], b[j] * vj[4 * m + e], ua);
             }
         }
         // C W and C U: MFMA (j, e) pairs tokens (8j + e, 8j + 4 + e), which is register
@@ -358,12 +370,33 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaParams P) {
                 cu = mfma_f32(ca[e], ua[4 * j + e], cu);
             }
         }
-        float *wt = P.w + tile * (kBlk * kDim), *qt = P.qp + tile * (kBlk * kDim);
+        // This wave's dims of K, W~ and Q' in the order the apply waves hold them: lane (n =
+        // lane % 16, g = lane / 16) of wave w takes token 16tt + n, dims 32w + 16mt + 4g ..+3
+        // of W~ and Q', tokens 16tt + 4g ..+3 of dim 32w + 16mt + n of K, at
+        // [w][tt][mt][lane][4]: every load there is 1 KB on end. K once a key head, by its
+        // even value head. W~ and Q' change order through this wave's own columns of ks and qs,
+        // which no other wave reads any more, so there is no barrier.
+        const int n = lane & 15, g = lane >> 4, at = wave * 1024 + 4 * lane;
+        if (!(head & 1)) {
+            float *kt = P.kf + ((size_t)blk * (kVHeads / 2) + kh) * (kBlk * kDim) + at;
+#pragma unroll
+            for (int f = 0; f < 4; f++) {
+                const float *k = ks + (16 * (f >> 1) + 4 * g) * kPad4 + 32 * wave + 16 * (f & 1) + n;
+                st4(kt + 256 * f, f4{k[0], k[kPad4], k[2 * kPad4], k[3 * kPad4]});
+            }
+        }
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const int t = 8 * (i >> 2) + 4 * h + (i & 3);
-            wt[t * kDim + dcol] = tl[t] * wa[i];
-            qt[t * kDim + dcol] = gs[t] * qs[t * kPad4 + dcol] - cw[i];
+            ks[t * kPad4 + dcol] = tl[t] * wa[i];
+            qs[t * kPad4 + dcol] = gs[t] * qs[t * kPad4 + dcol] - cw[i];
+        }
+        float *wt = P.w + tile * (kBlk * kDim) + at, *qt = P.qp + tile * (kBlk * kDim) + at;
+#pragma unroll
+        for (int f = 0; f < 4; f++) {
+            const int row = (16 * (f >> 1) + n) * kPad4 + 32 * wave + 16 * (f & 1) + 4 * g;
+            st4(wt + 256 * f, ld4(ks + row));
+            st4(qt + 256 * f, ld4(qs + row));
         }
         // U~ and C U in the apply blocks' layout (value row c = 16 rg + n, token
         // t = 16 tt + 4 g + i at [rg][tt][g][n][i]): registers 4q..4q+3 are four
@@ -379,179 +412,210 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(DeltaParams P) {
     }
 }
 
-// ---- chunkwise apply: one block per (head, 16 value rows), 256 blocks of 5 waves. Waves
-// 0..3 compute; wave w holds the state's key dims 32w..32w+31 as S^T in two 16x16 MFMA
-// accumulators (register i of lane l: dim 32w + 16mt + 4(l/16) + i, value row l%16). With
-// v_mfma_f32_16x16x4_f32 the k index of a product is the lane group l/16, so the k-steps
-// are chosen to take the state, or D~ (same layout), as the B operand straight from
-// registers: step (mt, i) covers dims 32w + 16mt + 4g + i (g = 0..3), and its A operands
-// are four consecutive floats of an LDS row (one 128-bit read per four MFMAs).
+// ---- chunkwise apply: one block per (head, 16 value rows), 256 blocks of 4 waves. Wave w
+// holds the state's key dims 32w..32w+31 as S^T in two 16x16 MFMA accumulators (register i
+// of lane l: dim 32w + 16mt + 4(l/16) + i, value row l%16). With v_mfma_f32_16x16x4_f32 the
+// k index of a product is the lane group l/16, so the k-steps are chosen to take the state,
+// or D~ (same layout), as the B operand straight from registers: step (mt, i) covers dims
+// 32w + 16mt + 4g + i (g = 0..3), and its A operands are four consecutive floats of a row.
 //
-// Wave 4 only copies: a block's operands (W~, Q', K rows, the block's U~ and CU, the
-// factors: 53 KB) go global -> LDS directly (global_load_lds), double-buffered, the next
-// block's while the current one computes. The copies pass the CU's address unit at about
-// 64 bytes a clock, so a wave issuing them stalls for most of a block; a wave of their own
-// keeps those stalls off the MFMA waves. Rows of 128 floats are stored with 16-byte piece
-// p of row t at slot p ^ (t & 31), so both the 128-bit reads of a row segment and the
-// 32-bit reads of a key column are conflict-free. Rows past the chunk's end read the
-// chunk's last token: their W~, U~, Q' and CU rows are zero, so they add nothing to the
-// state or to the stored rows.
-struct ApplySet {
-    float w[kBlk * kDim], q[kBlk * kDim], k[kBlk * kDim];
-    float u[kBlk * kApplyRows], cu[kBlk * kApplyRows];   // [tt][g][n][i], as prepare writes them
-    float f[2 * kBlk];                                    // (g, tail) per token
+// The walk over the blocks is serial, so a block's latency is what counts. Each lane reads
+// every operand it needs exactly once, and no two waves read the same W~, Q' or K element:
+// they go global -> registers, two blocks ahead (two stages, each refilled as soon as it is
+// consumed), in the order that prepare laid them out for that (1 KB on end a load), with
+// nothing staged through LDS. LDS holds only the waves' partial products, in two alternating
+// buffers, so that a block has a single barrier. Only W~ S^T and the state update are on the
+// chain: Q' S^T runs while the partial sums of W~ S^T travel through LDS, and its own partial
+// sums are added up, and the rows stored, one block later, between the update's MFMAs.
+//
+// 2,048 tokens: 108 us with the operands staged through LDS by four copy waves and two
+// barriers a block; 103 with register stages but row-major operands (16-row gathers of 64
+// bytes, keys in single words: with no loads at all that form took 88); 84-89 now. The
+// MFMAs alone, 48 a block and SIMD at 32 cycles, take about 47.
+struct ApplyStage {
+    f4 w[2][2], q[2][2];      // [tt][mt]: token 16tt + n, dims 32w + 16mt + 4g ..+3
+    f4 k[2][2];               // [tt][mt]: tokens 16tt + 4g ..+3, dim 32w + 16mt + n
+    f4 u[2];                  // [tt]: tokens 16tt + 4g ..+3 of value row n
+    dih_f32x2 cu;             // this wave's quarter of the output: two tokens of value row n
+    float glast;
 };
 
-DIH_DEV int slot128(int t, int p) { return 4 * (p ^ (t & 31)); }
+// Which operands a lane takes; with block bases in scalar registers the walk spends hardly any
+// vector instructions on addresses.
+struct ApplyLane {
+    uint32_t frag, u, cu, out;   // offsets (floats) from a block's W~, Q' or K, its U~, CU, rows
+    int ot, oi, head, rg;
+};
 
 DIH_DEV f4 mfma16(float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-// A quarter of a block's copies, by copy wave c: row pairs 4c..4c+3 of W~, Q' and K, one
-// half of U~ (c = 0, 1) or CU (c = 2, 3); copy wave 0 also the 64 factors.
-DIH_DEV void copy_block(ApplySet &S, const DeltaParams &P, int blk, int head, int kh, int rg, int c, int lane) {
-    const int base = blk * kBlk, valid = min(kBlk, P.tokens - base);
-    const size_t tile = (size_t)blk * kVHeads + head;
-    const float *wt = P.w + tile * (kBlk * kDim), *qt = P.qp + tile * (kBlk * kDim);
+DIH_DEV size_t apply_tile(const ApplyLane &L, int blk) { return ((size_t)blk * kVHeads + L.head) * (kBlk * kDim); }
+
+// A tile of W~, Q' or keys, [tt][mt] of this lane
+DIH_DEV void load_tile(f4 (&x)[2][2], const float *tile, const ApplyLane &L) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int pair = 4 * c + i, t = 2 * pair + (lane >> 5), p = (lane & 31) ^ (t & 31);
-        to_lds<16>(wt + t * kDim + 4 * p, S.w + 2 * pair * kDim);
-        to_lds<16>(qt + t * kDim + 4 * p, S.q + 2 * pair * kDim);
-        to_lds<16>(P.conv + (size_t)(base + min(t, valid - 1)) * kRowLen + kK + kh * kDim + 4 * p,
-                   S.k + 2 * pair * kDim);
+    for (int f = 0; f < 4; f++) x[f >> 1][f & 1] = ld4(tile + (L.frag + 256 * f));
+}
+
+DIH_DEV void load_rest(ApplyStage &S, const ApplyLane &L, const DeltaParams &P, int blk) {
+    const int valid = min(kBlk, P.tokens - blk * kBlk);
+    load_tile(S.k, P.kf + ((size_t)blk * (kVHeads / 2) + (L.head >> 1)) * (kBlk * kDim), L);
+    const float *u = P.u + apply_tile(L, blk) + L.rg * (kBlk * kApplyRows);
+    S.u[0] = ld4(u + L.u);
+    S.u[1] = ld4(u + (L.u + 256));
+    S.glast = P.factors[((size_t)blk * kVHeads + L.head) * (2 * kBlk) + 2 * (valid - 1)];
+}
+
+DIH_DEV void load_cu(ApplyStage &S, const ApplyLane &L, const DeltaParams &P, int blk) {
+    S.cu = *reinterpret_cast<const dih_f32x2 *>(P.cu + apply_tile(L, blk) + L.rg * (kBlk * kApplyRows) + L.cu);
+}
+
+struct ApplyParts {
+    float w[4][2][64 * 4], q[4][2][64 * 4];   // [wave][tt][lane * 4 + register]
+};
+
+// out = CU + the waves' sum of Q' S^T, this wave's quarter: token tile wave / 2, registers
+// 2 (wave & 1) and 2 (wave & 1) + 1. Stored through a buffer of the block's `rows` rows, which
+// drops what lies past them: no branch splits the walk.
+DIH_DEV void store_out(const ApplyParts &part, const ApplyLane &L, const DeltaParams &P, dih_f32x2 cu, int blk,
+                       int rows, int lane) {
+    const dih_f32x2 *p = reinterpret_cast<const dih_f32x2 *>(&part.q[0][L.ot][lane * 4 + L.oi]);
+    const dih_f32x2 o = ((p[0] + p[256]) + (p[512] + p[768])) + cu;
+    constexpr int kRowBytes = kVHeads * kDim * 4;
+    const auto buffer = __builtin_amdgcn_make_buffer_rsrc(P.out + (size_t)blk * (kBlk * kVHeads * kDim), 0,
+                                                          rows * kRowBytes, 0x00027000);
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[0]), buffer, 4 * L.out, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[1]), buffer, 4 * L.out + kRowBytes, 0, 0);
+}
+
+// Asks the scheduler for `N` MFMAs, each followed by some vector instructions and global loads.
+template <int N, int VALU, int LOADS>
+DIH_DEV void interleave() {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, VALU, 0);
+        if (LOADS) __builtin_amdgcn_sched_group_barrier(0x020, LOADS, 0);
     }
-    const int half = c & 1;
-    const float *src = (c < 2 ? P.u : P.cu) + tile * (kBlk * kDim) + rg * (kBlk * kApplyRows) + 256 * half;
-    to_lds<16>(src + 4 * lane, (c < 2 ? S.u : S.cu) + 256 * half);
-    if (c == 0) to_lds<4>(P.factors + tile * (2 * kBlk) + lane, S.f);
 }
 
-// The block's partial products of the four waves: D~ needs all of W~ S^T (eight 128-bit
-// reads: wave w2, token tile tt at byte offset 1024 (2 w2 + tt)), out one quarter of
-// Q' S^T (four 64-bit reads 2 KB apart).
-DIH_DEV void part_sums(const float *p1, const float *p2, f4 &d0, f4 &d1, dih_f32x2 &o) {
-    d0 = (ld4(p1) + ld4(p1 + 512)) + (ld4(p1 + 1024) + ld4(p1 + 1536));
-    d1 = (ld4(p1 + 256) + ld4(p1 + 768)) + (ld4(p1 + 1280) + ld4(p1 + 1792));
-    const dih_f32x2 *q = reinterpret_cast<const dih_f32x2 *>(p2);
-    o = (q[0] + q[256]) + (q[512] + q[768]);
-}
-
-// One block on a compute wave, from the set `S` the copy wave filled.
-DIH_DEV void apply_block(const ApplySet &S, float (&part)[2][4][2][64 * 4], f4 (&st)[2], const DeltaParams &P,
-                         int blk, int head, int rg, int wave, int lane) {
-    const int n = lane & 15, g = lane >> 4;
-    const int base = blk * kBlk, valid = min(kBlk, P.tokens - base);
-
-    // partial (over this wave's dims) W~ S^T and Q' S^T, token tiles tt: C[m = token][n = row];
-    // all eight operand reads first (the scheduler would otherwise wait on each pair just
-    // before its MFMAs)
-    f4 wa[2][2], qa[2][2];
+// Block blk from stage S, which it refills for block blk + 2 (past the end: the last block
+// again, unused). `done` holds the partial sums of block blk - 1 and R, its stage, its CU
+// values; they are refilled for block blk + 1 here. (A stage's values are never copied: a copy
+// would wait for the load just issued.)
+DIH_DEV void apply_block(ApplyStage &S, ApplyStage &R, ApplyParts &now, const ApplyParts &done, f4 (&st)[2],
+                         const ApplyLane &L, const DeltaParams &P, int blk, int wave, int lane) {
+    const int next = min(blk + 2, P.nblocks - 1);
+    f4 p[2];
+    // partial (over this wave's dims) W~ S^T, token tiles tt: C[m = token][n = row]
+    p[0] = p[1] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int tt = 0; tt < 2; tt++)
+    for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-        for (int mt = 0; mt < 2; mt++) {
-            const int t = 16 * tt + n, at = t * kDim + slot128(t, 8 * wave + 4 * mt + g);
-            wa[tt][mt] = ld4(S.w + at);
-            qa[tt][mt] = ld4(S.q + at);
-        }
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int tt = 0; tt < 2; tt++) p[tt] = mfma16(S.w[tt][mt][i], st[mt][i], p[tt]);
+#pragma unroll
+    for (int tt = 0; tt < 2; tt++) st4(&now.w[wave][tt][lane * 4], p[tt]);
     __builtin_amdgcn_sched_barrier(0);
-    f4 p1[2], p2[2];
+    barrier_no_fence();
+    __builtin_amdgcn_sched_barrier(0);
+    // D~ = U~ - the waves' sum of W~ S^T, the first half of Q' S^T running during the reads, the
+    // second between the sums (an MFMA occupies its pipe for 32 cycles, a wave for 4)
+    f4 part[2][4], d[2];
 #pragma unroll
-    for (int tt = 0; tt < 2; tt++) {
-        p1[tt] = f4{0.f, 0.f, 0.f, 0.f};
-        p2[tt] = p1[tt];
+    for (int tt = 0; tt < 2; tt++)
 #pragma unroll
-        for (int mt = 0; mt < 2; mt++)
+        for (int w = 0; w < 4; w++) part[tt][w] = ld4(&now.w[w][tt][lane * 4]);
+    __builtin_amdgcn_sched_barrier(0);
+    p[0] = p[1] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                p1[tt] = mfma16(wa[tt][mt][i], st[mt][i], p1[tt]);
-                p2[tt] = mfma16(qa[tt][mt][i], st[mt][i], p2[tt]);
-            }
-    }
-    // the state update's key operands, read ahead of the barrier: step (tt, i) covers tokens
-    // 16tt + 4g + i, tile mt dims 32w + 16mt + n
-    float ka[2][2][4];
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int tt = 0; tt < 2; tt++) p[tt] = mfma16(S.q[tt][0][i], st[0][i], p[tt]);
+    load_tile(S.w, P.w + apply_tile(L, next), L);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int tt = 0; tt < 2; tt++) p[tt] = mfma16(S.q[tt][1][i], st[1][i], p[tt]);
+#pragma unroll
+    for (int tt = 0; tt < 2; tt++) d[tt] = S.u[tt] - ((part[tt][0] + part[tt][1]) + (part[tt][2] + part[tt][3]));
+    st[0] *= S.glast;
+    interleave<8, 5, 0>();
+    __builtin_amdgcn_sched_barrier(0);
+    // S^T <- g_last S^T + K^T D~: step (tt, i) covers tokens 16tt + 4g + i (the two state
+    // tiles' chains in turn: two chains keep the MFMA pipe full). Between them the previous
+    // block's rows and the next loads.
+    st[1] *= S.glast;
 #pragma unroll
     for (int tt = 0; tt < 2; tt++)
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int mt = 0; mt < 2; mt++) {
-                const int t = 16 * tt + 4 * g + i, dim = 32 * wave + 16 * mt + n;
-                ka[tt][mt][i] = S.k[t * kDim + slot128(t, dim >> 2) + (dim & 3)];
-            }
+            for (int mt = 0; mt < 2; mt++) st[mt] = mfma16(S.k[tt][mt][i], d[tt][i], st[mt]);
+    store_out(done, L, P, R.cu, max(blk - 1, 0), blk ? kBlk : 0, lane);
 #pragma unroll
-    for (int tt = 0; tt < 2; tt++) {
-        st4(&part[0][wave][tt][lane * 4], p1[tt]);
-        st4(&part[1][wave][tt][lane * 4], p2[tt]);
-    }
-    wait_lgkm0();
-    barrier_no_fence();
-    // D~ = U~ - sum_waves(W~ S^T) in full; out = CU + sum_waves(Q' S^T) for this wave's
-    // quarter: token tile wave / 2, registers 2 (wave & 1) and 2 (wave & 1) + 1
-    const int ot = wave >> 1, oi = 2 * (wave & 1);
-    f4 s0, s1;
-    dih_f32x2 o;
-    part_sums(&part[0][0][0][lane * 4], &part[1][0][ot][lane * 4 + oi], s0, s1, o);
-    const f4 d0 = ld4(S.u + lane * 4) - s0, d1 = ld4(S.u + 256 + lane * 4) - s1;
-    o += *reinterpret_cast<const dih_f32x2 *>(S.cu + 256 * ot + lane * 4 + oi);
-    float *ob = P.out + (size_t)(base + 16 * ot + 4 * g + oi) * (kVHeads * kDim) + head * kDim + rg * kApplyRows + n;
-    if (16 * ot + 4 * g + oi < valid) ob[0] = o[0];
-    if (16 * ot + 4 * g + oi + 1 < valid) ob[kVHeads * kDim] = o[1];
-
-    // S^T <- g_last S^T + K^T D~: step (tt, i) covers tokens 16tt + 4g + i (the two state
-    // tiles' chains in turn: two chains keep the MFMA pipe full)
-    const float glast = S.f[2 * (valid - 1)];
-#pragma unroll
-    for (int mt = 0; mt < 2; mt++) st[mt] *= glast;
-#pragma unroll
-    for (int tt = 0; tt < 2; tt++) {
-        const f4 d = tt ? d1 : d0;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++) st[mt] = mfma16(ka[tt][mt][i], d[i], st[mt]);
-    }
+    for (int tt = 0; tt < 2; tt++) st4(&now.q[wave][tt][lane * 4], p[tt]);
+    load_tile(S.q, P.qp + apply_tile(L, next), L);
+    load_cu(R, L, P, min(blk + 1, P.nblocks - 1));
+    load_rest(S, L, P, next);
+    interleave<16, 4, 2>();
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 // Blocks: XCD x (block b runs on XCD b % 8) takes value heads 2x, 2x + 1, 2x + 16, 2x + 17
 // (two key heads), eight row groups each, so the blocks sharing a head's W~, Q' and K
-// tiles share one L2. Two barriers a block: after the partial products (the sums need all
-// four), and at its end (the copy wave's copies of the next block have landed, and the
-// compute waves are done with this block's set and partial sums).
-__global__ __launch_bounds__(512, 1) void delta_apply_kernel(DeltaParams P) {
-    __shared__ __align__(16) ApplySet sets[2];
-    __shared__ __align__(16) float part[2][4][2][64 * 4];
-    lds_escape(sets, part);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+// tiles share one L2.
+//
+// A partial-sum buffer is written before barrier b (W~ S^T) and after it (Q' S^T), read
+// after barrier b and after barrier b + 1, and next written after barrier b + 1 by a wave
+// that has passed it: the reads of W~ S^T were waited for before that barrier. Its Q' S^T
+// part is read after barrier b + 1 and next written after barrier b + 2.
+__global__ __launch_bounds__(256, 2) void delta_apply_kernel(DeltaParams P) {
+    __shared__ __align__(16) ApplyParts part[2];
+    lds_escape(part);
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 15, g = lane >> 4;
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, hl = slot >> 3, rg = slot & 7;
-    const int head = 2 * xcd + (hl & 1) + 16 * (hl >> 1), kh = head >> 1;
+    const int head = 2 * xcd + (hl & 1) + 16 * (hl >> 1);
+    ApplyLane L;
+    L.ot = wave >> 1;
+    L.oi = 2 * (wave & 1);
+    L.head = head;
+    L.rg = rg;
+    L.frag = wave * 1024 + 4 * lane;
+    L.u = 4 * lane;
+    L.cu = 256 * L.ot + 4 * lane + L.oi;
+    L.out = (16 * L.ot + 4 * g + L.oi) * (kVHeads * kDim) + head * kDim + rg * kApplyRows + n;
 
-    // (barriers without the memory fence: __syncthreads() would make the copy wave wait for
-    // its copies at the mid-block barrier, and the compute waves for their row stores)
-    if (wave >= 4) {
-        copy_block(sets[0], P, 0, head, kh, rg, wave - 4, lane);
-        wait_vm<0>();
-        barrier_no_fence();
-        for (int blk = 0; blk < P.nblocks; blk++) {
-            if (blk + 1 < P.nblocks) copy_block(sets[(blk + 1) & 1], P, blk + 1, head, kh, rg, wave - 4, lane);
-            barrier_no_fence();
-            wait_vm<0>();
-            barrier_no_fence();
-        }
-    } else {
-        float *sbase =
-            P.state + ((size_t)head * kDim + rg * kApplyRows + (lane & 15)) * kDim + 32 * wave + 4 * (lane >> 4);
-        f4 st[2] = {ld4(sbase), ld4(sbase + 16)};
-        barrier_no_fence();
-        for (int blk = 0; blk < P.nblocks; blk++) {
-            apply_block(sets[blk & 1], part, st, P, blk, head, rg, wave, lane);
-            barrier_no_fence();
-        }
-        st4(sbase, st[0]);
-        st4(sbase + 16, st[1]);
-        if (blockIdx.x < kRowLen / 256) roll_history(P, blockIdx.x * 256 + tid);
+    float *sbase = P.state + ((size_t)head * kDim + rg * kApplyRows + n) * kDim + 32 * wave + 4 * g;
+    f4 st[2] = {ld4(sbase), ld4(sbase + 16)};
+    const int last = P.nblocks - 1, rows = P.tokens - last * kBlk;
+    ApplyStage a, b;
+    load_tile(a.w, P.w + apply_tile(L, 0), L);
+    load_tile(a.q, P.qp + apply_tile(L, 0), L);
+    load_rest(a, L, P, 0);
+    load_tile(b.w, P.w + apply_tile(L, min(1, last)), L);
+    load_tile(b.q, P.qp + apply_tile(L, min(1, last)), L);
+    load_rest(b, L, P, min(1, last));
+    load_cu(a, L, P, 0);
+    b.cu = dih_f32x2{0.f, 0.f};
+#pragma clang loop unroll(disable)
+    for (int blk = 0; blk < last; blk += 2) {
+        apply_block(a, b, part[0], part[1], st, L, P, blk, wave, lane);
+        apply_block(b, a, part[1], part[0], st, L, P, blk + 1, wave, lane);
     }
+    if (last & 1) {
+        barrier_no_fence();
+        store_out(part[1], L, P, b.cu, last, rows, lane);
+    } else {
+        apply_block(a, b, part[0], part[1], st, L, P, last, wave, lane);
+        barrier_no_fence();
+        store_out(part[0], L, P, a.cu, last, rows, lane);
+    }
+    st4(sbase, st[0]);
+    st4(sbase + 16, st[1]);
+    if (blockIdx.x < kRowLen / 256) roll_history(P, blockIdx.x * 256 + tid);
 }
 
 }  // namespace
@@ -560,14 +624,14 @@ bool launch_delta_rule(const DeltaArgs &a, hipStream_t s, char *error, int capac
     DeltaParams P;
     P.conv = a.conv; P.decay = a.decay; P.beta = a.beta; P.raw = a.raw;
     P.state = a.state; P.history = a.history; P.out = a.out;
-    P.w = a.w; P.u = a.u; P.qp = a.qp; P.cu = a.cu; P.factors = a.factors;
+    P.w = a.w; P.u = a.u; P.qp = a.qp; P.cu = a.cu; P.factors = a.factors; P.kf = a.kf;
     P.tokens = a.tokens;
     P.nblocks = (a.tokens + kBlk - 1) / kBlk;
     if (!a.chunked) {
         DIH_LAUNCH(delta_seq_kernel, dim3(kVHeads * kDim / 16), dim3(256), 0, s, P);
         return hip_ok(hipGetLastError(), error, capacity, "delta launch");
     }
-    if (!P.w || !P.u || !P.qp || !P.cu || !P.factors) {
+    if (!P.w || !P.u || !P.qp || !P.cu || !P.factors || !P.kf) {
         set_error(error, capacity, "Chunkwise delta rule needs its scratch buffers");
         return false;
     }
@@ -575,7 +639,7 @@ bool launch_delta_rule(const DeltaArgs &a, hipStream_t s, char *error, int capac
     DIH_LAUNCH(delta_prepare_kernel, dim3(kVHeads, P.nblocks), dim3(256), 0, s, P);
     if (!hip_ok(hipGetLastError(), error, capacity, "delta prepare launch")) return false;
     prof_stage("delta_apply");
-    DIH_LAUNCH(delta_apply_kernel, dim3(kVHeads * (kDim / kApplyRows)), dim3(512), 0, s, P);
+    DIH_LAUNCH(delta_apply_kernel, dim3(kVHeads * (kDim / kApplyRows)), dim3(256), 0, s, P);
     return hip_ok(hipGetLastError(), error, capacity, "delta apply launch");
 }
 

@@ -115,6 +115,22 @@ def test_delta_rule_other_path(device, mode, T, path):
     _check(got_out, got_state, outs[:T], states[T])
 
 
+@pytest.mark.parametrize("T", [1, 32, 33, 64, 79, 96, 97, 130, 159])
+def test_delta_chunkwise_keeps_to_its_rows(device, T):
+    """One to five blocks of 32 tokens, the last one full, ragged or a single token: every
+    row of the chunk is right, and the rows behind it are not written."""
+    conv, a, b, state, _, _ = _oracle(3)
+    want_out, want_state = orc.delta_rule_f64(state, conv, a, b, T)
+    d_state = torch.from_numpy(np.ascontiguousarray(state)).cuda()
+    out = torch.full((T + 40, 4096), 7.5, device="cuda")
+    dc, da, db = (torch.from_numpy(np.ascontiguousarray(x[:T])).cuda() for x in (conv, a, b))
+    dh.delta_rule(device, d_state, torch.zeros((3, 8192), device="cuda"), dc, da, db,
+                  torch.zeros((T, 8192), device="cuda"), out, T, path=2)
+    torch.cuda.synchronize()
+    _check(out[:T].cpu().numpy(), d_state.cpu().numpy(), want_out, want_state)
+    assert bool((out[T:] == 7.5).all())
+
+
 def test_delta_rule_carries_state(device):
     """Two chunkwise calls of 100 and 65 tokens equal the recurrence over 165."""
     conv, a, b, state, _, _ = _oracle(0)
