@@ -455,7 +455,7 @@ DIH_DEV void multiply_tile(uint32_t vs, uint32_t ks, const uint32_t (&pw)[8], co
 template <bool RESTARTS>
 __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
     __shared__ __align__(16) uint16_t ks[3][kKeys * kDim];
-    __shared__ __align__(16) uint16_t vs[3][kKeys * kDim];
+    __shared__ __align__(16) uint16_t vs[4][kKeys * kDim];   // (the fourth: zeros)
     lds_escape(ks, vs);
 
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, r = lane & 31, h = lane >> 5;
@@ -471,6 +471,9 @@ __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
     if (kstart >= kend) return;
 
     const int wtok0 = tok0 + 4 * wave;
+#pragma unroll
+    for (int i = 0; i < kKeys * kDim / (8 * 512); i++)
+        *reinterpret_cast<uint4 *>(&vs[3][8 * (t + 512 * i)]) = make_uint4(0, 0, 0, 0);
     dih_bf16x8 qreg[16];
     load_queries(qreg, P, wtok0 + (r >> 3), wtok0 + (r >> 3) < P.tokens, kh * kGroup + (r & 7), h);
     RowState st;
@@ -482,6 +485,11 @@ __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
 
     const uint16_t *kbase = P.keys + kh * kDim, *vbase = P.values + kh * kDim;
     const int ntile = (kend - kstart + kKeys - 1) / kKeys;
+    // Tiles up to the wave's last visible key. Those behind have probabilities of 0 for all of the
+    // wave's rows, but 0 times a NaN or an infinity of a later token's value row would still be
+    // NaN: the wave multiplies them as zeros (a slot's number, where a branch around the
+    // products costs 288 spilled registers).
+    const int visible = (P.position + min(wtok0 + 3, P.tokens - 1) - kstart + kKeys) / kKeys;
     dih_f32x16 s;
     uint32_t pw[8];
     // Copy i of a tile's keys (or values) by this wave: rows 4 * wave + 2i and the next one, from
@@ -517,7 +525,7 @@ __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
         return l;
     };
     // (every wave takes part in every tile: rows that see none of its keys have masked scores,
-    // which leave their state and accumulators as they are)
+    // which leave their state as it is; for the products see `visible`)
     auto soften = [&](int j) {
         const int kb = kstart + j * kKeys;
         const bool full = kb + kKeys - 1 <= P.position + wtok0 && kb + kKeys <= kend;
@@ -543,10 +551,14 @@ __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
     int s0 = 0, s1 = 1, s2 = 2;   // slots of tiles j, j + 1, j + 2
     if (wave >= 4) flip();        // the second group runs one phase behind
     for (int j = 0; j < ntile; j++) {
+        // (formed ahead of the softmax: scalar work between a flip and the first operand read
+        // is time on the chain)
+        uint32_t vtile = vs_lds + (uint32_t)(j < visible ? s0 : 3) * kSlot;
+        asm volatile("" : "+s"(vtile));
         soften(j);
         flip();
         const int l = fresh();
-        multiply_tile(vs_lds + (uint32_t)s0 * kSlot, ks_lds + (uint32_t)s1 * kSlot, pw, qreg, acc, s, l, [&](int i) {
+        multiply_tile(vtile, ks_lds + (uint32_t)s1 * kSlot, pw, qreg, acc, s, l, [&](int i) {
             if (i < 2) copy(vfirst, vs_lds + (uint32_t)s2 * kSlot, false, j + 2, i, l);
             else copy(kfirst, ks_lds + (uint32_t)s0 * kSlot, true, j + 3, i - 2, l);
         });

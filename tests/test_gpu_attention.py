@@ -200,6 +200,29 @@ def test_attention_eight_wave_edges(device, inputs, position, count):
     assert np.all(np.isnan(got[count:]))
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("position,count,at,partition", [
+    (16, 64, 24, 0), (47, 64, 20, 0), (17, 33, 30, 0), (4016, 64, 24, 32), (2992, 100, 56, 128)])
+def test_attention_nonfinite_later_value(device, inputs, position, count, at, partition, bad):
+    """A non-finite value row of token `at` stays out of the waves (4 tokens) whose last token comes
+    before that key's 32-key tile; the tokens from `at` on see it."""
+    I = inputs
+    vb = I.vb.copy()
+    vb[position + at] = orc.f32_to_bf16_bits(np.full(512, bad, np.float32))
+    out = torch.full((256, 4096), 7.0, device="cuda")
+    dh.attention(device, I.dq, I.dk, torch.from_numpy(vb.view(np.int16)).cuda(), I.draw, out, position, count,
+                 partition=partition)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    clean = ((position + at) // 32 * 32 - position) // 4 * 4
+    assert clean >= 8
+    want = orc.attention_f64(I.q[:clean], I.k, I.v, I.raw[:clean], position,
+                             partition=dh.attention_partition(position, count, partition))
+    _check(got[:clean], want)
+    assert not np.isfinite(got[at:count]).any()
+    assert (got[count:] == 7.0).all()
+
+
 @pytest.mark.parametrize("position", [0, 31, 32, 96, 127, 128, 129, 255, 1000, 8191])
 def test_attention_decode_positions(device, inputs, position):
     """One decode token (the decode kernels: 128-key blocks of four 32-key tiles, after the
