@@ -285,8 +285,9 @@ int dih_grouped_qmm(void *context, void *matrix, void *up_matrix, int tokens, co
 /* Dense batched projection (p_gemv dense path, gpu_prefill.mm:603-620, prefill_bf16.mm:7-53):
  * Y[t][r] = sum_c w(0,r,c)*X[t][c]. Up to 4 tokens: a batched f32 GEMV; longer chunks: the
  * fused MFMA qmm with bf16 operands, short ones split over K (the partial sums live in the
- * context, a fixed 32 MiB for each of the first four streams that call; other streams, and
- * streams under capture, run unsplit); from 1024 tokens (512 for matrices of up to 4096 rows),
+ * context: 32 MiB for its own stream and up to three of 32 MiB for all others, allocated at
+ * the first such call; a call on another stream waits for the previous one with the same
+ * planes; calls under capture run unsplit); from 1024 tokens (512 for matrices of up to 4096 rows),
  * where it is the faster, the matrix dequantized once into bf16 context scratch (2*R*C bytes),
  * then the library's bf16 MFMA GEMM. bf16 operands, f32 accumulation in every MFMA form; the
  * order of the f32 sums depends on the form. x bf16

@@ -151,18 +151,54 @@ static hipStream_t pick(Context *c, void *stream) {
     return stream ? static_cast<hipStream_t>(stream) : c->stream;
 }
 
-// Split-K planes for a dense call on `s`, or null: a stream past the slots, or one under
-// capture (a graph's kernels would keep the slot of the capturing stream and could replay
-// beside that stream's own calls).
-static float *dense_planes(Context *c, hipStream_t s) {
-    if (!c->planes) return nullptr;
+// A slot of split-K planes for a dense call on `s`, or null: no memory, or a stream under
+// capture (a graph's kernels would keep the slot and could replay beside its next caller).
+// The context's own stream has slot 0 to itself: one stream for the context's life, whose
+// calls follow each other. A caller's handle does not identify a stream: hipStreamPerThread
+// is another one in every thread, and the handle of a destroyed stream comes back while its
+// work may still run. The other slots are therefore ordered by events: `s` waits for the
+// slot's previous sum, whoever queued it. Among them the handle only picks the slot whose wait
+// is most likely over: its own, then an unused one, then the one used longest ago.
+static Context::PlaneSlot *dense_planes(Context *c, hipStream_t s) {
+    if (c->plane_failed) return nullptr;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return nullptr;
-    int i = 0;
-    while (i < c->plane_used && c->plane_stream[i] != s) i++;
-    if (i == Context::kPlaneSlots) return nullptr;
-    if (i == c->plane_used) c->plane_stream[c->plane_used++] = s;
-    return reinterpret_cast<float *>(c->planes + (size_t)i * Context::kPlaneBytes);
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (st != hipStreamCaptureStatusNone) return nullptr;
+    Context::PlaneSlot *p = &c->plane[0];
+    if (s != c->stream) {
+        p = &c->plane[1];
+        for (Context::PlaneSlot &q : c->plane) {
+            if (&q == &c->plane[0]) continue;
+            if (q.last && q.stream == s) {
+                p = &q;
+                break;
+            }
+            if (q.last < p->last) p = &q;
+        }
+    }
+    bool ok = true;
+    if (!p->mem) {
+        // (another thread's stream may be under capture, where an allocation in the default
+        // mode would end that capture)
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        ok = hipMalloc(reinterpret_cast<void **>(&p->mem), Context::kPlaneBytes) == hipSuccess;
+        if (!ok) p->mem = nullptr;
+        if (ok && p != &c->plane[0]) ok = hipEventCreateWithFlags(&p->done, hipEventDisableTiming) == hipSuccess;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    if (ok && p->last && p->done) ok = hipStreamWaitEvent(s, p->done, 0) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();
+        c->plane_failed = true;
+        return nullptr;
+    }
+    p->stream = s;
+    p->last = ++c->plane_calls;
+    return p;
 }
 
 static bool stage(Matrix *m, size_t in_floats, size_t out_floats, char *error, int capacity) {
@@ -245,11 +281,6 @@ __attribute__((visibility("default"))) void *dih_quant_create_configured(int res
         delete c;
         return nullptr;
     }
-    // (without the planes dense calls run unsplit)
-    if (hipMalloc(reinterpret_cast<void **>(&c->planes), Context::kPlaneSlots * Context::kPlaneBytes) != hipSuccess) {
-        c->planes = nullptr;
-        (void)hipGetLastError();
-    }
     return c;
 }
 
@@ -263,7 +294,10 @@ __attribute__((visibility("default"))) void dih_quant_destroy(void *p) {
     (void)hipStreamSynchronize(c->stream);
     for (auto &s : c->ws)
         if (s.ptr) (void)hipFree(s.ptr);
-    if (c->planes) (void)hipFree(c->planes);
+    for (auto &p : c->plane) {
+        if (p.mem) (void)hipFree(p.mem);
+        if (p.done) (void)hipEventDestroy(p.done);
+    }
     for (auto &e : c->prof_pool) (void)hipEventDestroy(e);
     (void)hipEventDestroy(c->start);
     (void)hipEventDestroy(c->stop);
@@ -1160,9 +1194,17 @@ __attribute__((visibility("default"))) int dih_dense(void *ctx, void *matrix, in
         return ok ? 0 : -1;
     }
     QmmArgs a;
-    a.part = dense_planes(c, s);
-    a.part_bytes = a.part ? Context::kPlaneBytes : 0;
-    a.plan = dense_plan(m, tokens, a.part_bytes);
+    Context::PlaneSlot *slot = nullptr;
+    a.plan = dense_plan(m, tokens, Context::kPlaneBytes, s != c->stream);
+    if (!a.plan.gemm && a.plan.ksplit > 1) {
+        slot = dense_planes(c, s);
+        if (slot) {
+            a.part = slot->mem;
+            a.part_bytes = Context::kPlaneBytes;
+        } else {
+            a.plan = dense_plan(m, tokens, 0, false);
+        }
+    }
     if (a.plan.gemm) {
         bool ok = launch_dense_gemm(c, m, tokens, static_cast<const uint16_t *>(x), y, y_dtype == DIH_BF16, s,
                                     error, capacity);
@@ -1172,6 +1214,10 @@ __attribute__((visibility("default"))) int dih_dense(void *ctx, void *matrix, in
     a.m0 = m; a.tokens = tokens; a.dense = 1; a.x = static_cast<const uint16_t *>(x); a.in_mode = 0;
     a.y = y; a.y_bf16 = y_dtype == DIH_BF16;
     bool ok = launch_qmm(a, s, error, capacity);
+    if (slot && slot->done && !hip_ok(hipEventRecord(slot->done, s), error, capacity, "split-K event")) {
+        c->plane_failed = true;   // (the slot's next caller could not wait)
+        ok = false;
+    }
     prof_mark(c, s, "dense_qmm");
     return ok ? 0 : -1;
 }

@@ -70,14 +70,20 @@ struct Context {
     int prof_used = 0;                        // events taken from the pool since reset
     // named scratch
     Scratch ws[32];
-    // Split-K planes of dih_dense, one slot per stream (the first kPlaneSlots streams that
-    // ask; others run unsplit), so that dense calls on different streams of one context stay
-    // independent of each other. Allocated with the context, freed with it.
+    // Split-K planes of dih_dense (dense_planes in abi.hip): slot 0 for the context's own
+    // stream, the others shared out to the streams that callers bring, so that dense calls on
+    // different streams of one context seldom wait for each other. A slot's 32 MiB are
+    // allocated at its first call and freed with the context.
     static constexpr int kPlaneSlots = 4;
     static constexpr size_t kPlaneBytes = (size_t)32 << 20;
-    char *planes = nullptr;
-    hipStream_t plane_stream[kPlaneSlots] = {};
-    int plane_used = 0;
+    struct PlaneSlot {
+        float *mem = nullptr;
+        hipStream_t stream = nullptr;   // the last caller's (slots past 0)
+        hipEvent_t done = nullptr;      // after the last sum (slots past 0)
+        uint64_t last = 0;              // number of that call (0: never used)
+    } plane[kPlaneSlots];
+    uint64_t plane_calls = 0;
+    bool plane_failed = false;          // no memory for a slot: dense calls run unsplit
     // this device's copy of the fixed scratch array of dih_moe_decode_noalloc (its device
     // address, looked up once per device), or null with the lookup's error
     void *noalloc = nullptr;
@@ -189,8 +195,9 @@ struct DensePlan {
     bool gemm = false;
     int nt = 0, ksplit = 1;
 };
-// The fastest by estimate; part_bytes: split-K planes available (0: no ranges).
-DensePlan dense_plan(const Matrix *m, int tokens, size_t part_bytes);
+// The fastest by estimate; part_bytes: split-K planes available (0: no ranges); ordered: their
+// use is ordered by events.
+DensePlan dense_plan(const Matrix *m, int tokens, size_t part_bytes, bool ordered);
 
 struct QmmArgs {
     // routed matrices (gate or down) and optional up for the gated kernel

@@ -876,9 +876,12 @@ bool qmm_wide_gated(const Matrix *gate, int tokens) {
 // projections, 5 and 8 bits, 16 to 1023 tokens; median error 5 %, and the plan it picks is
 // 0.5 % behind the best one on average, 7 % at worst). n blocks of nt 32-token tiles run on
 // each CU, `resident` at a time; a K step of c resident blocks takes the larger of one
-// block's latency and c times its issue time. Ranges add the sum pass: its launch and the
-// planes' write and read.
-static double dense_cost(int bits, size_t items, int nt, int steps, int ksplit, size_t plane_bytes) {
+// block's latency and c times its issue time. Ranges add the sum pass: its launch, the
+// planes' write and read and, with planes ordered by events (`ordered`), the event's record
+// and its gap (split on the context's stream, split on another, unsplit: 61 tokens of a
+// 2048 x 4096 matrix 11.5, 16.9 and 23.6 us, 16 tokens of 8192 x 2048 10.2, 14.9 and 13.0,
+// 64 tokens of 512 x 2048 9.4, 15.7 and 13.1: the last two run unsplit there).
+static double dense_cost(int bits, size_t items, int nt, int steps, int ksplit, size_t plane_bytes, bool ordered) {
     constexpr int kResident[2][5] = {{0, 4, 3, 2, 1}, {0, 3, 2, 2, 1}};   // by LDS: 5-bit, 8-bit
     const int resident = kResident[bits == 8][nt];
     const double slow = bits == 8 ? 1.0 : 1.1, latency = 0.2 + 0.111 * nt, issue = 0.185 + 0.054 * nt;
@@ -886,7 +889,7 @@ static double dense_cost(int bits, size_t items, int nt, int steps, int ksplit, 
     const auto round = [&](size_t c) { return 0.755 + slow * steps * std::max(latency, issue * (double)c); };
     double t = 4.3 + (double)(n / resident) * round(resident);
     if (n % resident) t += round(n % resident);
-    return ksplit > 1 ? t + 0.78 + (double)ksplit * (double)plane_bytes * 2.0 / 5.0e6 : t;
+    return ksplit > 1 ? t + (ordered ? 9.0 : 0.78) + (double)ksplit * (double)plane_bytes * 2.0 / 5.0e6 : t;
 }
 
 // The same for one dequantization pass and the bf16 GEMM of gemm.hip: a round of 256 tiles
@@ -913,7 +916,7 @@ static bool qmm_in_range(const Matrix *m, int tokens) {
 // tiles whose blocks share a CU, so that one's dequantization overlaps another's MFMAs and
 // the last round is finer (8192 x 2048: 128 tokens 23.7 -> 13.7 us, 700 tokens 48.1 -> 29.7
 // us; 512 x 2048 at 1023 tokens 17.6 us as a GEMM -> 12.6 us).
-DensePlan dense_plan(const Matrix *m, int tokens, size_t part_bytes) {
+DensePlan dense_plan(const Matrix *m, int tokens, size_t part_bytes, bool ordered) {
     DensePlan best;
     // (shorter chunks never need the bf16 copy of the weights)
     const bool may_gemm = tokens >= 1024 || (tokens >= 512 && m->rows <= 4096);
@@ -929,7 +932,7 @@ DensePlan dense_plan(const Matrix *m, int tokens, size_t part_bytes) {
         const size_t plane = items * 128 * 32 * (size_t)nt * 4;
         if (chunks > 0xffff || (nt > 1 && tokens <= 32 * (nt - 1))) continue;
         for (int k = 1; k <= windows && (k == 1 || k * plane <= part_bytes); k *= 2) {
-            const double c = dense_cost(m->bits, items, nt, 4 * ((windows + k - 1) / k), k, plane);
+            const double c = dense_cost(m->bits, items, nt, 4 * ((windows + k - 1) / k), k, plane, ordered);
             if (best.nt == 0 || c < cost) {
                 cost = c;
                 best.nt = nt;

@@ -6,6 +6,7 @@ tolerance) against the fp64 oracle of the reference's dequantize-then-matmul; ti
 bounds are asserted where the arithmetic allows (noted per test).
 """
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -809,9 +810,9 @@ def test_dense_split_ranges(device, bits, rows, columns, T):
 
 
 def test_dense_short_chunks_on_streams_and_in_graphs():
-    """Split-K planes belong to a stream: calls on more streams than a context holds planes
-    for (the last ones run unsplit), queued beside each other on one context, and a call
-    captured in a graph as the context's first (nothing allocated) all give the f64 product."""
+    """Calls on more streams than a context holds split-K planes for, queued beside each other on
+    one context, and a call captured in a graph as the context's first (unsplit, nothing
+    allocated) all give the f64 product."""
     rng = np.random.default_rng(61)
     T, rows, columns = 61, 512, 4096
     host = orc.random_matrix(rng, 1, rows, columns, 8)
@@ -844,6 +845,58 @@ def test_dense_short_chunks_on_streams_and_in_graphs():
                 assert orc.rel_err(y.cpu().numpy(), w) < 1e-4
             assert orc.rel_err(yg.cpu().numpy(), want[0]) < 1e-4
         del g
+        m.dispose()
+
+
+def test_dense_planes_on_per_thread_and_many_streams():
+    """A stream handle does not identify a stream: hipStreamPerThread (handle 2) is another one
+    in every thread. Threads that serialize their calls on one context and pass it, and callers
+    with more streams than there are plane slots, all run split over K and give the bits of
+    the same call on the context's own stream."""
+    rng = np.random.default_rng(62)
+    T, rows, columns, threads = 61, 2048, 4096, 3
+    with dh.QuantizedHip() as dev:
+        m = upload(dev, orc.random_matrix(rng, 1, rows, columns, 8))
+        xs = [dev_bf16(orc.f32_to_bf16_bits(rng.normal(size=(T, columns)).astype(np.float32))) for _ in range(8)]
+        ys = [torch.zeros((T, rows), device="cuda") for _ in xs]
+        want = [torch.zeros((T, rows), device="cuda") for _ in xs]
+        dh.set_profiling(dev, True)
+        for x, y in zip(xs, want):
+            dh.dense(dev, m, T, x, y)
+        streams = [torch.cuda.Stream() for _ in xs]
+        torch.cuda.synchronize()
+        assert dh.profile_read(dev)["dense_qmm"][1] == 2 * len(xs)   # the ranges and their sum
+        dh.set_profiling(dev, True)
+        for st, x, y in zip(streams, xs, ys):
+            dh.dense(dev, m, T, x, y, stream=st)
+        torch.cuda.synchronize()
+        assert dh.profile_read(dev)["dense_qmm"][1] == 2 * len(xs)
+        dh.set_profiling(dev, False)
+        for y, w in zip(ys, want):
+            assert torch.equal(y, w)
+            y.zero_()
+        torch.cuda.synchronize()
+        lock, gate, errors = threading.Lock(), threading.Barrier(threads), []
+
+        def work(i):
+            try:
+                gate.wait()
+                for _ in range(50):
+                    with lock:
+                        dh.dense(dev, m, T, xs[i], ys[i], stream=2)   # hipStreamPerThread
+                torch.cuda.synchronize()   # (the thread's stream ends with the thread)
+            except Exception as e:
+                errors.append(e)
+
+        pool = [threading.Thread(target=work, args=(i,)) for i in range(threads)]
+        for t in pool:
+            t.start()
+        for t in pool:
+            t.join()
+        torch.cuda.synchronize()
+        assert not errors, errors
+        for y, w in zip(ys[:threads], want):
+            assert torch.equal(y, w)
         m.dispose()
 
 
