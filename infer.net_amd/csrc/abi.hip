@@ -151,8 +151,17 @@ static hipStream_t pick(Context *c, void *stream) {
     return stream ? static_cast<hipStream_t>(stream) : c->stream;
 }
 
-// A slot of split-K planes for a dense call on `s`, or null: no memory, or a stream under
-// capture (a graph's kernels would keep the slot and could replay beside its next caller).
+// Whether `s` is under capture (also when that cannot be told).
+static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
+// A slot of split-K planes for a dense call on `s`, or null without memory for one. Not for
+// streams under capture: a graph's kernels would keep the slot and could replay beside its next
+// caller.
 // The context's own stream has slot 0 to itself: one stream for the context's life, whose
 // calls follow each other. A caller's handle does not identify a stream: hipStreamPerThread
 // is another one in every thread, and the handle of a destroyed stream comes back while its
@@ -161,12 +170,6 @@ static hipStream_t pick(Context *c, void *stream) {
 // is most likely over: its own, then an unused one, then the one used longest ago.
 static Context::PlaneSlot *dense_planes(Context *c, hipStream_t s) {
     if (c->plane_failed) return nullptr;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (st != hipStreamCaptureStatusNone) return nullptr;
     Context::PlaneSlot *p = &c->plane[0];
     if (s != c->stream) {
         p = &c->plane[1];
@@ -317,12 +320,16 @@ __attribute__((visibility("default"))) uint64_t dih_quant_residency_bytes(void *
 
 __attribute__((visibility("default"))) void dih_quant_residency_prepare(void *) {}
 
+static bool matrix_shape_ok(int experts, int rows, int columns, int bits) {
+    return experts >= 1 && experts <= 256 && rows >= 1 && columns >= 64 && columns <= 8192 && columns % 64 == 0 &&
+           (bits == 5 || bits == 8);
+}
+
 __attribute__((visibility("default"))) void *dih_quant_matrix_create(void *ctx, int experts, int rows,
                                                                      int columns, int bits, int group,
                                                                      char *error, int capacity) {
     Context *c = as_ctx(ctx);
-    if (!c || experts < 1 || experts > 256 || rows < 1 || columns < 64 || columns > 8192 ||
-        (bits != 5 && bits != 8) || group != 64 || columns % 64) {
+    if (!c || !matrix_shape_ok(experts, rows, columns, bits) || group != 64) {
         set_error(error, capacity, "Unsupported quantized matrix shape");
         return nullptr;
     }
@@ -1168,6 +1175,28 @@ __attribute__((visibility("default"))) int dih_grouped_qmm(void *ctx, void *matr
     return ok ? 0 : -1;
 }
 
+// Dispatch policy (p_gemv, gpu_prefill.mm:603-620, picks GEMV kernels below 64 tokens):
+// up to kDenseGemvTokens tokens run as one batched GEMV launch (each token a slot of
+// expert 0; it multiplies unrounded weights, so where it ends is also a rounding point),
+// longer chunks on bf16 MFMAs as dense_plan chooses.
+static constexpr int kDenseGemvTokens = 4;
+
+__attribute__((visibility("default"))) int dih_dense_plan(int rows, int columns, int bits, int tokens, int planes,
+                                                          int *tiles, int *ranges) {
+    if (tokens < 1 || !tiles || !ranges || planes < 0 || planes > 2 || !matrix_shape_ok(1, rows, columns, bits))
+        return -1;
+    *tiles = 0;
+    *ranges = 1;
+    if (tokens <= kDenseGemvTokens) return 0;
+    Matrix m;
+    m.experts = 1; m.rows = rows; m.columns = columns; m.bits = bits;
+    const DensePlan plan = dense_plan(&m, tokens, planes ? Context::kPlaneBytes : 0, planes == 1);
+    if (plan.gemm) return 2;
+    *tiles = plan.nt;
+    *ranges = plan.ksplit;
+    return 1;
+}
+
 __attribute__((visibility("default"))) int dih_dense(void *ctx, void *matrix, int tokens, const void *x, void *y,
                                                      int y_dtype, void *stream, char *error, int capacity) {
     Context *c = as_ctx(ctx);
@@ -1180,11 +1209,6 @@ __attribute__((visibility("default"))) int dih_dense(void *ctx, void *matrix, in
     if (!sync_matrix(m, error, capacity)) return -1;
     hipStream_t s = pick(c, stream);
     ProfScope prof_scope(c);
-    // Dispatch policy (p_gemv, gpu_prefill.mm:603-620, picks GEMV kernels below 64 tokens):
-    // up to kDenseGemvTokens tokens run as one batched GEMV launch (each token a slot of
-    // expert 0; it multiplies unrounded weights, so where it ends is also a rounding point),
-    // longer chunks on bf16 MFMAs as dense_plan chooses.
-    constexpr int kDenseGemvTokens = 4;
     if (tokens <= kDenseGemvTokens) {
         QmvSeg sg = seg_of(m);
         sg.count = tokens; sg.x = x; sg.x_bf16 = 1; sg.x_slot_stride = m->columns;
@@ -1195,7 +1219,10 @@ __attribute__((visibility("default"))) int dih_dense(void *ctx, void *matrix, in
     }
     QmmArgs a;
     Context::PlaneSlot *slot = nullptr;
-    a.plan = dense_plan(m, tokens, Context::kPlaneBytes, s != c->stream);
+    const bool graph = capturing(s);
+    a.plan = dense_plan(m, tokens, graph ? 0 : Context::kPlaneBytes, s != c->stream);
+    // (the GEMM's weight copy cannot grow under capture)
+    if (graph && a.plan.nt && c->ws[S_W16].bytes < (size_t)m->rows * m->columns * 2) a.plan.gemm = false;
     if (!a.plan.gemm && a.plan.ksplit > 1) {
         slot = dense_planes(c, s);
         if (slot) {

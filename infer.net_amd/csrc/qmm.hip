@@ -872,6 +872,17 @@ bool qmm_wide_gated(const Matrix *gate, int tokens) {
            (size_t)tokens * 8 > (size_t)48 * (size_t)std::max(1, gate->experts);
 }
 
+// Widest block of a dense launch, in 32-token tiles. (Four leave one block a CU, whose
+// dequantization and MFMAs take turns: the fastest form of 5 % of 3,618 measured
+// shapes and chunks, by 3 % on average.)
+constexpr int kDenseTiles = 3;
+
+// Blocks of nt 32-token tiles that a CU's LDS holds.
+static int dense_resident(int bits, int nt) {
+    constexpr int kResident[2][kDenseTiles + 1] = {{0, 4, 3, 2}, {0, 3, 2, 2}};
+    return kResident[bits == 8][nt];
+}
+
 // The estimate dense_plan minimizes, in us, fitted to 770 measured launches (four model
 // projections, 5 and 8 bits, 16 to 1023 tokens; median error 5 %, and the plan it picks is
 // 0.5 % behind the best one on average, 7 % at worst). n blocks of nt 32-token tiles run on
@@ -882,8 +893,7 @@ bool qmm_wide_gated(const Matrix *gate, int tokens) {
 // 2048 x 4096 matrix 11.5, 16.9 and 23.6 us, 16 tokens of 8192 x 2048 10.2, 14.9 and 13.0,
 // 64 tokens of 512 x 2048 9.4, 15.7 and 13.1: the last two run unsplit there).
 static double dense_cost(int bits, size_t items, int nt, int steps, int ksplit, size_t plane_bytes, bool ordered) {
-    constexpr int kResident[2][5] = {{0, 4, 3, 2, 1}, {0, 3, 2, 2, 1}};   // by LDS: 5-bit, 8-bit
-    const int resident = kResident[bits == 8][nt];
+    const int resident = dense_resident(bits, nt);
     const double slow = bits == 8 ? 1.0 : 1.1, latency = 0.2 + 0.111 * nt, issue = 0.185 + 0.054 * nt;
     const size_t n = (items * (size_t)ksplit + 255) / 256;
     const auto round = [&](size_t c) { return 0.755 + slow * steps * std::max(latency, issue * (double)c); };
@@ -892,16 +902,35 @@ static double dense_cost(int bits, size_t items, int nt, int steps, int ksplit, 
     return ksplit > 1 ? t + (ordered ? 9.0 : 0.78) + (double)ksplit * (double)plane_bytes * 2.0 / 5.0e6 : t;
 }
 
-// The same for one dequantization pass and the bf16 GEMM of gemm.hip: a round of 256 tiles
-// costs its shape's time a 64-column step, a partial one 60 % of that plus its share.
-static double dense_gemm_cost(const Matrix *m, int tokens) {
+// From 512 tokens on the choice between the fused launch and the GEMM has estimates of its own,
+// of a whole pass among others: dense_cost above ranks fused launches, but is 10 to 40 % low
+// where blocks run in several rounds. Fitted to 12,294 passes of the fused form (19 shapes, 5
+// and 8 bits, 400 to 8192 tokens, bf16 and f32 rows; median error 4 %) and 2,136 of the GEMM
+// (4 %). The stores count by the element where rows are not whole quads (fused) or 16-byte
+// pieces of bf16 (GEMM).
+static double dense_fused_pass(const Matrix *m, int tokens, size_t items, int nt, int steps, int ksplit,
+                               size_t plane_bytes) {
+    const double slow = m->bits == 8 ? 1.0 : 1.057, latency = 0.257 + 0.088 * nt, issue = 0.164 + 0.091 * nt;
+    const int resident = dense_resident(m->bits, nt);
+    const size_t n = (items * (size_t)ksplit + 255) / 256;
+    const auto round = [&](size_t c) { return slow * steps * std::max(latency, issue * (double)c); };
+    double t = 9.1 + (double)(n / resident) * round(resident);
+    if (n % resident) t += round(n % resident);
+    if (ksplit > 1) t += 2.0 + (double)ksplit * (double)plane_bytes * 2.0 / 7.2e6;
+    return t + (double)tokens * m->rows * 1e-6 * (m->rows % 4 ? 2.66 : 0.475);
+}
+
+// One dequantization pass and the bf16 GEMM of gemm.hip: a round of 256 tiles costs its shape's
+// time a 64-column step, a partial one after it nearly as much.
+static double dense_gemm_pass(const Matrix *m, int tokens) {
     int bm, bn;
     gemm_tile(m->rows, tokens, bm, bn);
-    const double step = bm * bn >= 65536 ? 1.77 : bm * bn >= 32768 ? 1.1 : bm * bn >= 16384 ? 0.53 : 0.37;
+    const double step = bm * bn >= 65536 ? 1.44 : bm * bn >= 32768 ? 0.83 : bm * bn >= 16384 ? 0.50 : 0.32;
     const size_t tiles = (size_t)((m->rows + bm - 1) / bm) * (size_t)((tokens + bn - 1) / bn);
     double rounds = (double)(tiles / 256);
-    if (tiles % 256) rounds += tiles < 256 ? 1.0 : 0.6 + 0.4 * (double)(tiles % 256) / 256.0;
-    return 6.0 + (double)m->rows * m->columns * (m->bits / 8.0 + 2.0) / 5.3e6 + rounds * (m->columns / 64) * step;
+    if (tiles % 256) rounds += tiles < 256 ? 1.0 : 0.93 + 0.07 * (double)(tiles % 256) / 256.0;
+    return 12.15 + (double)m->rows * m->columns * (m->bits / 8.0 + 2.0) / 3.47e6 + rounds * (m->columns / 64) * step +
+           (double)tokens * m->rows * 1e-6 * (m->rows % 8 ? 2.07 : 0.58);
 }
 
 // Limits of the kernels' 32-bit offsets: an expert's weight rows (padded to whole 256-row
@@ -926,23 +955,28 @@ DensePlan dense_plan(const Matrix *m, int tokens, size_t part_bytes, bool ordere
     }
     const size_t row_tiles = (size_t)(m->rows + 127) / 128;
     const int windows = m->columns / 256;   // of four K steps
-    double cost = 0;
-    for (int nt = 1; nt <= 4; nt++) {
+    double cost = 0, pass = 0;
+    for (int nt = 1; nt <= kDenseTiles; nt++) {
         const size_t chunks = ((size_t)tokens + 32 * nt - 1) / (32 * nt), items = row_tiles * chunks;
         const size_t plane = items * 128 * 32 * (size_t)nt * 4;
         if (chunks > 0xffff || (nt > 1 && tokens <= 32 * (nt - 1))) continue;
         for (int k = 1; k <= windows && (k == 1 || k * plane <= part_bytes); k *= 2) {
-            const double c = dense_cost(m->bits, items, nt, 4 * ((windows + k - 1) / k), k, plane, ordered);
+            // (k ranges of whole windows may leave the last ones empty: they are not launched)
+            const int per = (windows + k - 1) / k, ranges = (windows + per - 1) / per;
+            const double c = dense_cost(m->bits, items, nt, 4 * per, ranges, plane, ordered);
             if (best.nt == 0 || c < cost) {
                 cost = c;
                 best.nt = nt;
-                best.ksplit = k;
+                best.ksplit = ranges;
+                if (may_gemm) pass = dense_fused_pass(m, tokens, items, nt, 4 * per, ranges, plane);
             }
         }
     }
-    // (5 % for the estimates' error: 2048 tokens of a 2048 x 4096 matrix take 44.4 us as a GEMM
-    // and 46.9 us fused, 1300 tokens 53.6 and 36.3 us)
-    best.gemm = may_gemm && (best.nt == 0 || dense_gemm_cost(m, tokens) < 1.05 * cost);
+    // The GEMM where it is the faster by estimate; 3 % are left to it for the estimates' errors.
+    // Over the fit's 1,220 cases from 512 tokens on, the launch taken is 11 % faster than the GEMM on average
+    // and behind it by more than 3 % in 15 (worst 9 %): 1280 tokens of a 2048 x 4096 8-bit
+    // matrix 61 us as a GEMM and 44 fused, 4096 tokens of 12288 x 2048 194 and 283.
+    best.gemm = may_gemm && (best.nt == 0 || dense_gemm_pass(m, tokens) < 1.03 * pass);
     return best;
 }
 
@@ -977,8 +1011,8 @@ static bool launch_dense_split(const QmmArgs &a, QmmParams P, hipStream_t s, cha
         DIH_LAUNCH((qmm_lds_kernel<B, false, N, 4, false, B == 5, N, 4>), grid, dim3(256), 0, s, P);   \
         found = true;                                                                                  \
     }
-    DIH_DENSE_CASE(8, 1) DIH_DENSE_CASE(8, 2) DIH_DENSE_CASE(8, 3) DIH_DENSE_CASE(8, 4)
-    DIH_DENSE_CASE(5, 1) DIH_DENSE_CASE(5, 2) DIH_DENSE_CASE(5, 3) DIH_DENSE_CASE(5, 4)
+    DIH_DENSE_CASE(8, 1) DIH_DENSE_CASE(8, 2) DIH_DENSE_CASE(8, 3)
+    DIH_DENSE_CASE(5, 1) DIH_DENSE_CASE(5, 2) DIH_DENSE_CASE(5, 3)
 #undef DIH_DENSE_CASE
     if (!found) {
         set_error(error, capacity, "Unsupported qmm configuration");

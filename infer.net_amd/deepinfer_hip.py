@@ -83,7 +83,7 @@ EXPORTS = [
     "dih_quant_batch", "dih_quant_matvec", "dih_quant_experts", "dih_quant_embedding",
     "dih_qmv", "dih_qmv_swiglu", "dih_lm_head", "dih_argmax", "dih_top8", "dih_build_groups",
     "dih_dequant_bf16", "dih_moe_decode", "dih_moe_prefill", "dih_moe_decode_norm", "dih_moe_decode_noalloc",
-    "dih_moe_prefill_norm", "dih_grouped_qmm", "dih_dense", "dih_attention",
+    "dih_moe_prefill_norm", "dih_grouped_qmm", "dih_dense", "dih_dense_plan", "dih_attention",
     "dih_attention_partition", "dih_delta_rule", "dih_delta_create", "dih_delta_destroy",
     "dih_delta_step", "dih_set_profiling",
     "dih_profile_read", "dih_version",
@@ -138,6 +138,7 @@ def load():
         "dih_moe_decode_noalloc": ([P, P, P, P, P, P, P, P, E, I], I),
         "dih_moe_prefill_norm": ([P, P, I, P, P, I, P, P, P, P, E, I], I),
         "dih_dense": ([P, P, I, P, P, I, P, E, I], I),
+        "dih_dense_plan": ([I, I, I, I, I, P, P], I),
         "dih_grouped_qmm": ([P, P, P, I, P, I, P, P, P, I, P, E, I], I),
         "dih_attention": ([P, P, I, P, P, I, P, I, P, I, I, I, I, P, E, I], I),
         "dih_attention_partition": ([I, I, I], I),
@@ -624,6 +625,16 @@ def dense(dev, m, tokens, x, y, y_dtype=F32, stream=None) -> None:
     err = _errbuf()
     _check(dev._lib.dih_dense(_ctx(dev), m.handle, tokens, _dp(x), _dp(y), y_dtype, _stream(stream), err, _ERR),
            err, ArgumentError)
+
+
+def dense_plan(rows, columns, bits, tokens, planes=2):
+    """(route, 32-token tiles a block, K ranges) of a dense() call (dih_dense_plan): route "gemv",
+    "fused" or "gemm"; planes 0: under capture, 1: on a caller's stream, 2: on the context's."""
+    tiles, ranges = ctypes.c_int(), ctypes.c_int()
+    route = load().dih_dense_plan(rows, columns, bits, tokens, planes, ctypes.byref(tiles), ctypes.byref(ranges))
+    if route < 0:
+        raise ArgumentError("Invalid dense projection arguments")
+    return ("gemv", "fused", "gemm")[route], tiles.value, ranges.value
 
 
 def attention(dev, q, keys, values, gate, out, position, tokens, partition=0, q_dtype=F32,

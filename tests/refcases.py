@@ -91,3 +91,24 @@ def stable_top8(values):
     """graph_checks.mm:67-68: sort by value descending, ties by index ascending."""
     order = np.lexsort((np.arange(values.size), -values.astype(np.float64)))
     return order[:8]
+
+
+# Dense projections (rows, columns, tokens) of short and medium chunks: K in one and several ranges,
+# whole and with a shorter last one, in each width of the blocks; rows past and off the
+# 128-row tiles and not whole float4, tokens past and off the 32-token tiles; the last two of the
+# first block are past the GEMM's first token count.
+DENSE_FUSED_SHAPES = [
+    (512, 2048, 5), (512, 2048, 32), (2048, 4096, 33), (2048, 4096, 64), (300, 2048, 65), (129, 4096, 96),
+    (1003, 2048, 97), (2048, 512, 128), (513, 1536, 129), (4100, 512, 160), (512, 8192, 193), (300, 2560, 300),
+    (8192, 512, 700), (512, 2048, 1300), (2048, 1024, 1500),
+    (8192, 2560, 5), (4099, 5120, 33), (2045, 5120, 129), (2500, 512, 400), (4100, 1024, 33), (2500, 4608, 65),
+    (129, 6656, 300)]
+
+# (bits, rows, columns, tokens, bf16 rows, the GEMM's block: rows x tokens): each block shape with
+# ragged row and token tiles, rows in and off 16-byte pieces.
+DENSE_GEMM_SHAPES = [
+    (8, 8200, 2048, 4100, True, (256, 256)), (8, 6001, 2048, 4100, True, (256, 256)),
+    (8, 6001, 1984, 4100, False, (256, 256)), (8, 2050, 4032, 4100, False, (256, 128)),
+    (8, 2051, 4032, 4100, True, (256, 128)), (5, 1000, 1024, 4096, True, (128, 128)),
+    (8, 1003, 1984, 4100, False, (128, 128)), (8, 300, 448, 1100, False, (128, 64)),
+    (5, 301, 1984, 1030, True, (128, 64))]

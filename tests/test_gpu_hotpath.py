@@ -706,22 +706,40 @@ def test_dense_matches_oracle(device, bits, rows, columns, T):
         m.dispose()
 
 
-@pytest.mark.parametrize("bits,rows,columns,T,y_bf16", [(8, 300, 512, 1024, False), (8, 2048, 4096, 512, True),
-                                                        (5, 1000, 2048, 1100, False), (5, 64, 256, 2048, True),
-                                                        (8, 4100, 1024, 512, False)])
-def test_dense_long_chunks_bf16_gemm(device, bits, rows, columns, T, y_bf16):
+def _dense_route(device, run):
+    """The route that dense() took in run(), by the launches it recorded."""
+    dh.set_profiling(device, True)
+    try:
+        run()
+        torch.cuda.synchronize()
+        launches = {name: count for name, (_, count) in dh.profile_read(device).items()}
+    finally:
+        dh.set_profiling(device, False)
+    if "dense_gemm" in launches:
+        assert launches == {"dense_dequant": 1, "dense_gemm": 1}
+        return "gemm"
+    assert set(launches) == {"dense_qmm"} and launches["dense_qmm"] in (1, 2)
+    return "split" if launches["dense_qmm"] == 2 else "fused"
+
+
+@pytest.mark.parametrize("bits,rows,columns,T,y_bf16,route", [
+    (8, 300, 512, 1024, False, "fused"), (8, 2048, 4096, 512, True, "split"), (5, 1000, 2048, 1100, False, "split"),
+    (5, 64, 256, 2048, True, "gemm"), (8, 4100, 1024, 512, False, "fused"),   # (past 4096 rows: from 1024 tokens)
+    (8, 300, 448, 1024, False, "gemm"), (8, 2048, 4032, 512, True, "gemm"), (8, 4096, 4096, 2048, True, "gemm")])
+def test_dense_long_chunks(device, bits, rows, columns, T, y_bf16, route):
     """Long chunks (1024 tokens and more, or 512 and more for matrices of up to 4096 rows)
-    run as one dequantization pass into bf16 and a bf16 GEMM with f32 accumulation (the
-    reference's BF16 dense path, prefill_bf16.mm:7-53): the result is the fp64 product of
-    the same bf16-rounded operands within fp32 accumulation error. (8, 4100, 1024, 512)
-    stays on the fused tile (more than 4096 rows at 512 tokens)."""
+    run fused or as one dequantization pass into bf16 and a bf16 GEMM with f32 accumulation
+    (the reference's BF16 dense path, prefill_bf16.mm:7-53), whichever is the faster: the
+    result is the fp64 product of the same bf16-rounded operands within fp32 accumulation
+    error."""
     rng = np.random.default_rng(rows * 7 + T)
     host = orc.random_matrix(rng, 1, rows, columns, bits)
     m = upload(device, host)
     try:
         xb = orc.f32_to_bf16_bits(rng.normal(size=(T, columns)).astype(np.float32))
         y = torch.zeros((T, rows), dtype=torch.int16 if y_bf16 else torch.float32, device="cuda")
-        dh.dense(device, m, T, dev_bf16(xb), y, y_dtype=dh.BF16 if y_bf16 else dh.F32)
+        assert _dense_route(device, lambda: dh.dense(device, m, T, dev_bf16(xb), y,
+                                                     y_dtype=dh.BF16 if y_bf16 else dh.F32)) == route
         # a second call (the scratch copy already sized) gives the same bits
         y2 = torch.zeros_like(y)
         dh.dense(device, m, T, dev_bf16(xb), y2, y_dtype=dh.BF16 if y_bf16 else dh.F32)
@@ -737,22 +755,23 @@ def test_dense_long_chunks_bf16_gemm(device, bits, rows, columns, T, y_bf16):
         m.dispose()
 
 
-@pytest.mark.parametrize("bits,rows,columns,T,y_bf16", [
-    (8, 8200, 2048, 4100, True),    # 256 x 256 tiles; ragged last row and token tiles
-    (8, 2050, 4096, 4100, False),   # 256 x 128 tiles; f32 rows not 16-byte aligned (element stores)
-    (5, 1000, 1024, 4096, True)])   # 128 x 128 tiles, 5-bit dequantization
-def test_dense_gemm_tile_shapes(device, bits, rows, columns, T, y_bf16):
+@pytest.mark.parametrize("bits,rows,columns,T,y_bf16,block", refcases.DENSE_GEMM_SHAPES + [
+    (8, 2050, 4096, 4100, False, None)])   # (the fused kernel's, off its 128-row tiles and float4 rows)
+def test_dense_gemm_tile_shapes(device, bits, rows, columns, T, y_bf16, block):
     """Every block shape of the library's bf16 GEMM (gemm_bf16_kernel, chosen by the tile
     count) against the fp64 product of the same bf16-rounded operands, with partial tiles at
-    both edges."""
+    the edges and rows in and off 16-byte pieces (element stores)."""
     rng = np.random.default_rng(rows + T)
     host = orc.random_matrix(rng, 1, rows, columns, bits)
     m = upload(device, host)
     try:
         xb = orc.f32_to_bf16_bits(rng.normal(size=(T, columns)).astype(np.float32))
-        y = torch.zeros((T, rows), dtype=torch.int16 if y_bf16 else torch.float32, device="cuda")
-        dh.dense(device, m, T, dev_bf16(xb), y, y_dtype=dh.BF16 if y_bf16 else dh.F32)
-        torch.cuda.synchronize()
+        y = torch.full((T + 1, rows), 7, dtype=torch.int16 if y_bf16 else torch.float32, device="cuda")
+        assert _dense_route(device, lambda: dh.dense(device, m, T, dev_bf16(xb), y,
+                                                     y_dtype=dh.BF16 if y_bf16 else dh.F32)) == \
+            ("gemm" if block else "fused")
+        assert (y[T] == 7).all()
+        y = y[:T]
         want = orc.dense_f64_blas(host, orc.bf16_bits_to_f32(xb), round_operands=True)
         if y_bf16:
             assert_rounded(host_bf16(y), want, rms(want) * 1e-2)
@@ -763,9 +782,9 @@ def test_dense_gemm_tile_shapes(device, bits, rows, columns, T, y_bf16):
 
 
 @pytest.mark.parametrize("bits,rows,columns,T", [(8, 16384, 512, 512), (5, 16400, 512, 520)])
-def test_dense_two_slab_tiles(device, bits, rows, columns, T):
-    """Dense launches with at least 256 (256-row tile, 128-token chunk) items run 256-row
-    tiles, two 32-row slabs a wave; ragged rows and tokens included."""
+def test_dense_many_row_tiles(device, bits, rows, columns, T):
+    """Chunks of matrices with 128 row tiles and more (several rounds of blocks); ragged rows and
+    tokens included."""
     rng = np.random.default_rng(rows + T)
     host = orc.random_matrix(rng, 1, rows, columns, bits)
     m = upload(device, host)
@@ -781,15 +800,11 @@ def test_dense_two_slab_tiles(device, bits, rows, columns, T):
 
 
 @pytest.mark.parametrize("bits", [8, 5])
-@pytest.mark.parametrize("rows,columns,T", [
-    (512, 2048, 5), (512, 2048, 32), (2048, 4096, 33), (2048, 4096, 64), (300, 2048, 65), (129, 4096, 96),
-    (1003, 2048, 97), (2048, 512, 128), (513, 1536, 129), (4100, 512, 160), (512, 8192, 193), (300, 2560, 300),
-    (8192, 512, 700), (512, 2048, 1300), (2048, 1024, 1500)])   # (the last two past the GEMM's first token count)
+@pytest.mark.parametrize("rows,columns,T", refcases.DENSE_FUSED_SHAPES)
 def test_dense_split_ranges(device, bits, rows, columns, T):
-    """Short dense chunks split K over work items and sum the planes: one to four 32-token
-    tiles a block, one and several ranges (the last one shorter: 1536 and 2560 columns), rows
-    past and off the 128-row tiles, rows not whole float4. f32 within fp32 accumulation of the
-    product of bf16-rounded operands, bf16 the same answer rounded once."""
+    """Short dense chunks split K over work items and sum the planes: one to three 32-token
+    tiles a block, one and several ranges, whole and with a shorter last one. f32 within fp32
+    accumulation of the product of bf16-rounded operands, bf16 the same answer rounded once."""
     rng = np.random.default_rng(rows + columns + T)
     host = orc.random_matrix(rng, 1, rows, columns, bits)
     m = upload(device, host)
@@ -797,7 +812,9 @@ def test_dense_split_ranges(device, bits, rows, columns, T):
         xb = orc.f32_to_bf16_bits(rng.normal(size=(T, columns)).astype(np.float32))
         y = torch.full((T + 1, rows), 7.0, dtype=torch.float32, device="cuda")
         yb = torch.full((T + 1, rows), 7, dtype=torch.int16, device="cuda")
-        dh.dense(device, m, T, dev_bf16(xb), y)
+        ranges = dh.dense_plan(rows, columns, bits, T)[2]
+        route = _dense_route(device, lambda: dh.dense(device, m, T, dev_bf16(xb), y))
+        assert route == ("split" if ranges > 1 else "fused")
         dh.dense(device, m, T, dev_bf16(xb), yb, y_dtype=dh.BF16)
         torch.cuda.synchronize()
         got = y.cpu().numpy()
@@ -845,6 +862,37 @@ def test_dense_short_chunks_on_streams_and_in_graphs():
                 assert orc.rel_err(y.cpu().numpy(), w) < 1e-4
             assert orc.rel_err(yg.cpu().numpy(), want[0]) < 1e-4
         del g
+        m.dispose()
+
+
+@pytest.mark.parametrize("rows,columns,T", [(8192, 4096, 1024), (512, 2048, 4096)])
+def test_dense_long_chunk_captured_first(rows, columns, T):
+    """A chunk that runs as the GEMM can be captured as its context's first call, where the weight
+    copy cannot be allocated (it then stays on the fused kernel), and after an eager call."""
+    rng = np.random.default_rng(T)
+    assert dh.dense_plan(rows, columns, 8, T, 0)[0] == "gemm"
+    host = orc.random_matrix(rng, 1, rows, columns, 8)
+    xb = orc.f32_to_bf16_bits(rng.normal(size=(T, columns)).astype(np.float32))
+    want = orc.dense_f64_blas(host, orc.bf16_bits_to_f32(xb), round_operands=True)
+    with dh.QuantizedHip() as dev:
+        m = upload(dev, host)
+        x, y, ye = dev_bf16(xb), torch.zeros((T, rows), device="cuda"), torch.zeros((T, rows), device="cuda")
+        torch.cuda.synchronize()
+        for _ in range(2):   # before and after the eager call
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g):
+                dh.dense(dev, m, T, x, y)
+            for _ in range(3):
+                y.zero_()
+                torch.cuda.synchronize()
+                g.replay()
+                torch.cuda.synchronize()
+                assert orc.rel_err(y.cpu().numpy(), want) < 1e-4
+                dh.dense(dev, m, T, x, ye)
+                torch.cuda.synchronize()
+                assert orc.rel_err(ye.cpu().numpy(), want) < 1e-4
+            del g
+        assert torch.equal(y, ye)
         m.dispose()
 
 
