@@ -297,11 +297,12 @@ int dih_dense(void *context, void *matrix, int tokens, const void *x, void *y, i
 
 /* How dih_dense runs `tokens` tokens of a [rows, columns] matrix: 0 the batched GEMV, 1 the fused
  * kernel with blocks of 32 * *tiles tokens (*tiles 0: the general fused kernel, columns not a
- * multiple of 512) and K in *ranges ranges, 2 the bf16 GEMM; -1 for arguments that dih_dense or
+ * multiple of 512) and 128 * *slabs rows and K in *ranges ranges, 2 the bf16 GEMM; -1 for arguments that dih_dense or
  * the matrix's creation refuses. `planes`: 0 a call under capture (which stays on the fused
  * kernel where the GEMM's weight copy would have to grow), 1 one on a caller's stream, 2 one
  * on the context's stream. Needs no device. */
-int dih_dense_plan(int rows, int columns, int bits, int tokens, int planes, int *tiles, int *ranges);
+int dih_dense_plan(int rows, int columns, int bits, int tokens, int planes, int *tiles, int *slabs,
+                   int *ranges);
 
 /* Causal GQA attention of `tokens` query tokens at cache positions position ..
  * position+tokens-1, with the output gate: the BF16 prefill attention and its partition

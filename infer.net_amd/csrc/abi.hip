@@ -1182,17 +1182,18 @@ __attribute__((visibility("default"))) int dih_grouped_qmm(void *ctx, void *matr
 static constexpr int kDenseGemvTokens = 4;
 
 __attribute__((visibility("default"))) int dih_dense_plan(int rows, int columns, int bits, int tokens, int planes,
-                                                          int *tiles, int *ranges) {
-    if (tokens < 1 || !tiles || !ranges || planes < 0 || planes > 2 || !matrix_shape_ok(1, rows, columns, bits))
+                                                          int *tiles, int *slabs, int *ranges) {
+    if (tokens < 1 || !tiles || !slabs || !ranges || planes < 0 || planes > 2 || !matrix_shape_ok(1, rows, columns, bits))
         return -1;
     *tiles = 0;
-    *ranges = 1;
+    *slabs = *ranges = 1;
     if (tokens <= kDenseGemvTokens) return 0;
     Matrix m;
     m.experts = 1; m.rows = rows; m.columns = columns; m.bits = bits;
     const DensePlan plan = dense_plan(&m, tokens, planes ? Context::kPlaneBytes : 0, planes == 1);
     if (plan.gemm) return 2;
     *tiles = plan.nt;
+    *slabs = plan.slabs;
     *ranges = plan.ksplit;
     return 1;
 }

@@ -189,11 +189,11 @@ bool launch_build_groups(const uint32_t *ids, int tokens, int experts, int with_
                          uint32_t *counts, uint32_t *routes, hipStream_t s, char *error, int capacity);
 
 // How a dense projection of more than the GEMV's tokens runs: dequantize + bf16 GEMM, or the
-// fused streaming kernel with `nt` 32-token tiles a block and K in `ksplit` ranges (nt 0: the
-// general fused kernel).
+// fused streaming kernel with `nt` 32-token tiles and 128 * `slabs` rows a block and K in
+// `ksplit` ranges (nt 0: the general fused kernel).
 struct DensePlan {
     bool gemm = false;
-    int nt = 0, ksplit = 1;
+    int nt = 0, slabs = 1, ksplit = 1;
 };
 // The fastest by estimate; part_bytes: split-K planes available (0: no ranges); ordered: their
 // use is ordered by events.

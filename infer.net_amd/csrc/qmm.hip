@@ -33,6 +33,7 @@
 // popular expert share that expert's weight rows in the XCD's L2. This replaces the
 // reference's atomic tile list and indirect dispatch (prefill_moe.mm:8-22) with a
 // deterministic order.
+#include <cmath>
 #include <type_traits>
 
 #include "dih_device.h"
@@ -365,9 +366,9 @@ __global__ __launch_bounds__(256, 2) void qmm_kernel(QmmParams P) {
 // Waves per SIMD the streaming kernel's registers are sized for: two blocks a CU where four
 // stages fit in half the LDS and the accumulators in the registers (four-wave blocks 256 a
 // lane, eight-wave ones 128), else one.
-template <int BITS, bool GATED, int NT, int NTC, bool SPLIT>
+template <int BITS, bool GATED, int NT, int NTC, bool SPLIT, int RS>
 constexpr int qmm_lds_waves() {
-    const bool two = 4 * ((GATED ? 2 : 1) * 128 * (64 * BITS / 8) + 32 * NT * 128) <= 80 * 1024 &&
+    const bool two = RS == 1 && 4 * ((GATED ? 2 : 1) * 128 * (64 * BITS / 8) + 32 * NT * 128) <= 80 * 1024 &&
                      (SPLIT ? NTC <= 2 : (GATED ? 2 : 1) * NTC <= 3);
     return (two ? 2 : 1) * (SPLIT ? 2 : 1);
 }
@@ -388,11 +389,15 @@ constexpr int qmm_lds_waves() {
 // ranges y is the planes' buffer: a block stores its f32 accumulators as they lie in
 // registers (1 KB a store instruction, where the tokens' rows would be 16-byte pieces) at its
 // (row tile, chunk) place of plane `range`, and splitk_sum_kernel adds the planes up.
-template <int BITS, bool GATED, int NT, int S, bool SPLIT, bool TL = false, int NTC = NT, int KS = 8>
-__global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, NTC, SPLIT>())) void qmm_lds_kernel(QmmParams P) {
+// RS (dense only): 32-row slabs a wave, so that a row tile is 128 * RS rows. Two slabs halve
+// the activation reads from LDS a row (every wave reads the whole token tile every step) and
+// take one range.
+template <int BITS, bool GATED, int NT, int S, bool SPLIT, bool TL = false, int NTC = NT, int KS = 8, int RS = 1>
+__global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, NTC, SPLIT, RS>())) void qmm_lds_kernel(QmmParams P) {
+    static_assert(RS == 1 || KS == 4, "two slabs a wave: dense launches only");
     static_assert(!SPLIT || GATED, "only the gated kernel splits its matrices over waves");
     static_assert(!TL || BITS == 5, "tile-major codes: 5-bit only");
-    constexpr int TR = 128;                  // rows per row tile
+    constexpr int TR = 128 * RS;             // rows per row tile
     constexpr int NW = SPLIT ? 8 : 4;        // waves per block
     static_assert(NTC >= 1 && NTC <= NT, "compute tiles within the copied route slots");
     constexpr int BN = 32 * NTC;             // routes per chunk (multiplied)
@@ -403,7 +408,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
     constexpr int WMAT = SPLIT ? 1 : NMAT;   // matrices one wave dequantizes
     constexpr int B_ST = BC * 128;
     constexpr int ST = NMAT * A_ST + B_ST;   // bytes per stage
-    constexpr int AQ = BITS == 8 ? 2 : 5;   // direct copies per wave per matrix per step
+    constexpr int AQ = (BITS == 8 ? 2 : 5) * RS;   // direct copies per wave per matrix per step
     constexpr int NBW = 4 * NT < NW ? 1 : 4 * NT / NW;   // activation copies (8 routes each) per wave
     static_assert(4 * NT < NW || NBW * NW == 4 * NT, "activation pieces split evenly over the waves");
     // (fewer pieces than waves: a piece is copied by two waves, the same bytes to the same place,
@@ -422,7 +427,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
 
     // the wave index is uniform: in a scalar register, LDS copy destinations need no readfirstlane
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
-    const int slab = wave & 3;                // 32-row slab of the 128-row tile
+    const int slab = wave & 3;                // 32 * RS rows of the tile
     const int mw = SPLIT ? wave >> 2 : 0;     // split: the matrix this wave computes
     // ---- work item (every wave derives it): physical block b runs logical item
     // L = xcd_item(b, items); L = chunk * rt_groups + row-tile group, a group being up to
@@ -493,11 +498,11 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
     for (int q = 0; q < AQ; q++) {
         if constexpr (BITS == 8) {
             const int rl = 16 * q + (lane >> 2), sl = lane & 3;
-            crow[q] = slab * 32 + rl;
+            crow[q] = slab * 32 * RS + rl;
             coff[q] = 16 * (sl ^ ((rl >> 2) & 3));
         } else {
             const int i = 64 * q + lane, rl = i / 10;
-            crow[q] = slab * 32 + rl;
+            crow[q] = slab * 32 * RS + rl;
             coff[q] = 4 * (i - rl * 10);
         }
     }
@@ -510,12 +515,15 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
     // and a FLAT load may read LDS, so it first waits for every LDS copy in flight (a full
     // drain of the copy pipeline once per eight steps).
     typedef __attribute__((address_space(1))) const wvec g_wvec;
-    auto win_load = [&](wvec (&sw)[2][2], int ti, int w) {
-        const size_t mrow = row_index(rt0 + ti, slab * 32 + r);
+    auto win_load = [&](wvec (&sw)[RS][2][2], int ti, int w) {
 #pragma unroll
-        for (int m = 0; m < WMAT; m++) {
-            sw[m][0] = *(g_wvec *)(psc[m + mw] + mrow * G + k0 + KS * w);
-            sw[m][1] = *(g_wvec *)(pbi[m + mw] + mrow * G + k0 + KS * w);
+        for (int rs = 0; rs < RS; rs++) {
+            const size_t mrow = row_index(rt0 + ti, slab * 32 * RS + 32 * rs + r);
+#pragma unroll
+            for (int m = 0; m < WMAT; m++) {
+                sw[rs][m][0] = *(g_wvec *)(psc[m + mw] + mrow * G + k0 + KS * w);
+                sw[rs][m][1] = *(g_wvec *)(pbi[m + mw] + mrow * G + k0 + KS * w);
+            }
         }
     };
 
@@ -596,9 +604,9 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
             for (int q = 0; q < AQ; q++) {
                 const char *src = wbase[mm] + (woff[q] + koff);
                 if constexpr (BITS == 8)
-                    to_lds<16>(src, base + m * A_ST + (slab * 32 + 16 * q) * 64);
+                    to_lds<16>(src, base + m * A_ST + (slab * 32 * RS + 16 * q) * 64);
                 else
-                    to_lds<4>(src, base + m * A_ST + slab * 32 * 40 + q * 256);
+                    to_lds<4>(src, base + m * A_ST + slab * 32 * RS * 40 + q * 256);
             }
         }
 #pragma unroll
@@ -611,18 +619,21 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
         }
     };
 
-    wvec win[2][2], win_next[2][2];
+    wvec win[RS][2][2], win_next[RS][2][2];
     if constexpr (KS == 4) win_load(win, 0, 0);   // (few steps: the first must not wait for the third's copies)
 #pragma unroll
     for (int st = 0; st < S - 1; st++) issue(st);
     if constexpr (KS != 4) win_load(win, 0, 0);
 
-    dih_f32x16 acc0[NTC], acc1[GATED && !SPLIT ? NTC : 1];
+    dih_f32x16 acc0[RS][NTC], acc1[GATED && !SPLIT ? NTC : 1];
     auto zero_acc = [&]() {
 #pragma unroll
-        for (int i = 0; i < NTC; i++) {
+        for (int rs = 0; rs < RS; rs++) {
 #pragma unroll
-            for (int k = 0; k < 16; k++) acc0[i][k] = 0.f;
+            for (int i = 0; i < NTC; i++) {
+#pragma unroll
+                for (int k = 0; k < 16; k++) acc0[rs][i][k] = 0.f;
+            }
         }
         if constexpr (GATED && !SPLIT) {
 #pragma unroll
@@ -647,12 +658,13 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
                 barrier_no_fence();
                 issue((u + S - 1) % S);
                 const unsigned char *base = stage_base(u % S);
-                // this step's weights -> bf16 A operands
-                dih_bf16x8 a[2][4];
+                // this step's weights -> bf16 A operands (a[rs * WMAT + m]: slab rs, matrix m)
+                dih_bf16x8 a[RS * 2][4];
 #pragma unroll
-                for (int m = 0; m < WMAT; m++) {
+                for (int rm = 0; rm < RS * WMAT; rm++) {
+                    const int rs = rm / WMAT, m = rm % WMAT;
                     Chunk<BITS> c;
-                    const int wr = slab * 32 + r;   // row within the tile
+                    const int wr = slab * 32 * RS + 32 * rs + r;   // row within the tile
                     if constexpr (BITS == 8) {
                         const int sw = (r >> 2) & 3;
                         const unsigned char *ra = base + (m + mw) * A_ST + wr * 64;
@@ -665,9 +677,9 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
 #pragma unroll
                         for (int k = 0; k < 5; k++) c.w[k] = ra[k];
                     }
-                    const uint32_t sbits = (win[m][0][u >> 1] >> (16 * (u & 1))) & 0xffffu;
-                    const uint32_t bbits = (win[m][1][u >> 1] >> (16 * (u & 1))) & 0xffffu;
-                    chunk_to_bf16<BITS>(c, bf16_to_f32(sbits), bf16_to_f32(bbits), a[m]);
+                    const uint32_t sbits = (win[rs][m][0][u >> 1] >> (16 * (u & 1))) & 0xffffu;
+                    const uint32_t bbits = (win[rs][m][1][u >> 1] >> (16 * (u & 1))) & 0xffffu;
+                    chunk_to_bf16<BITS>(c, bf16_to_f32(sbits), bf16_to_f32(bbits), a[rm]);
                 }
                 // MFMAs over all NT route tiles
                 const unsigned char *bb = base + NMAT * A_ST;
@@ -681,7 +693,9 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
                     }
 #pragma unroll
                     for (int i = 0; i < NTU; i++) {
-                        acc0[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][j], bx[i], acc0[i], 0, 0, 0);
+#pragma unroll
+                        for (int rs = 0; rs < RS; rs++)
+                            acc0[rs][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[rs * WMAT][j], bx[i], acc0[rs][i], 0, 0, 0);
                         if constexpr (GATED && !SPLIT)
                             acc1[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][j], bx[i], acc1[i], 0, 0, 0);
                     }
@@ -689,7 +703,10 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
             }
             if (more) {
 #pragma unroll
-                for (int m = 0; m < WMAT; m++) { win[m][0] = win_next[m][0]; win[m][1] = win_next[m][1]; }
+                for (int rm = 0; rm < RS * WMAT; rm++) {
+                    win[rm / WMAT][rm % WMAT][0] = win_next[rm / WMAT][rm % WMAT][0];
+                    win[rm / WMAT][rm % WMAT][1] = win_next[rm / WMAT][rm % WMAT][1];
+                }
             }
         }
 
@@ -698,7 +715,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
         // waves of the same slab through LDS (identical lane layouts), in the stage numbered as
         // the slab (a gated block has one row tile, so the stages are free once every wave's
         // copies have landed and its last operands are read); the up waves store.
-        if constexpr (KS == 4) {
+        if constexpr (KS == 4 && RS == 1) {
             if (P.ksplit > 1) {
                 const size_t at = ((size_t)(range * gridDim.x + rt0) * gridDim.z + blockIdx.z) * (TR * BN);
                 dih_f32x4 *dst = reinterpret_cast<dih_f32x4 *>(static_cast<float *>(P.y) + at) + slab * (NTC * 4 * 64) + lane;
@@ -707,8 +724,8 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
                     if (32 * i >= nvalid) break;
 #pragma unroll
                     for (int q = 0; q < 4; q++)
-                        dst[(i * 4 + q) * 64] = dih_f32x4{acc0[i][4 * q], acc0[i][4 * q + 1], acc0[i][4 * q + 2],
-                                                          acc0[i][4 * q + 3]};
+                        dst[(i * 4 + q) * 64] = dih_f32x4{acc0[0][i][4 * q], acc0[0][i][4 * q + 1],
+                                                          acc0[0][i][4 * q + 2], acc0[0][i][4 * q + 3]};
                 }
                 break;
             }
@@ -722,13 +739,15 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
 #pragma unroll
                 for (int i = 0; i < NTC; i++) {
 #pragma unroll
-                    for (int k = 0; k < 16; k++) xw[(i * 16 + k) * 64] = siluf_(acc0[i][k]);
+                    for (int k = 0; k < 16; k++) xw[(i * 16 + k) * 64] = siluf_(acc0[0][i][k]);
                 }
             }
             wait_lgkm0();
             barrier_no_fence();
         }
-        const int row_base = (rt0 + ti) * TR + slab * 32;
+#pragma unroll
+        for (int rs = 0; rs < RS; rs++) {
+        const int row_base = (rt0 + ti) * TR + slab * 32 * RS + 32 * rs;
 #pragma unroll
         for (int i = 0; i < NTC; i++) {
             const int n = 32 * i + r;
@@ -740,7 +759,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
                 float v[4];
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
-                    const float g = acc0[i][4 * q + k];
+                    const float g = acc0[rs][i][4 * q + k];
                     if constexpr (SPLIT) v[k] = xw[(i * 16 + 4 * q + k) * 64] * g;
                     else if constexpr (GATED) v[k] = siluf_(g) * acc1[i][4 * q + k];
                     else v[k] = g;
@@ -765,6 +784,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
                     }
                 }
             }
+        }
         }
         zero_acc();
     }
@@ -872,9 +892,8 @@ bool qmm_wide_gated(const Matrix *gate, int tokens) {
            (size_t)tokens * 8 > (size_t)48 * (size_t)std::max(1, gate->experts);
 }
 
-// Widest block of a dense launch, in 32-token tiles. (Four leave one block a CU, whose
-// dequantization and MFMAs take turns: the fastest form of 5 % of 3,618 measured
-// shapes and chunks, by 3 % on average.)
+// Widest block of the dense launches that share a CU, in 32-token tiles. (Four leave one block a
+// CU, whose dequantization and MFMAs take turns: see dense_one_round.)
 constexpr int kDenseTiles = 3;
 
 // Blocks of nt 32-token tiles that a CU's LDS holds.
@@ -908,6 +927,10 @@ static double dense_cost(int bits, size_t items, int nt, int steps, int ksplit, 
 // and 8 bits, 400 to 8192 tokens, bf16 and f32 rows; median error 4 %) and 2,136 of the GEMM
 // (4 %). The stores count by the element where rows are not whole quads (fused) or 16-byte
 // pieces of bf16 (GEMM).
+static double dense_store_pass(const Matrix *m, int tokens) {
+    return (double)tokens * m->rows * 1e-6 * (m->rows % 4 ? 2.66 : 0.475);
+}
+
 static double dense_fused_pass(const Matrix *m, int tokens, size_t items, int nt, int steps, int ksplit,
                                size_t plane_bytes) {
     const double slow = m->bits == 8 ? 1.0 : 1.057, latency = 0.257 + 0.088 * nt, issue = 0.164 + 0.091 * nt;
@@ -917,7 +940,32 @@ static double dense_fused_pass(const Matrix *m, int tokens, size_t items, int nt
     double t = 9.1 + (double)(n / resident) * round(resident);
     if (n % resident) t += round(n % resident);
     if (ksplit > 1) t += 2.0 + (double)ksplit * (double)plane_bytes * 2.0 / 7.2e6;
-    return t + (double)tokens * m->rows * 1e-6 * (m->rows % 4 ? 2.66 : 0.475);
+    return t + dense_store_pass(m, tokens);
+}
+
+// Blocks of four token tiles and one or two slabs, one a CU, where they take one round of the
+// GPU, which the narrower blocks then cross by a partial one. `pass`: the best of the others; the
+// wide form is taken from 8 % (one slab, 60 of 3,618 cases measured, 3.4 % faster on average) or
+// 5 % (two, 164 of 2,688, 9 %) below it, by the estimates' errors. One-slab blocks of up to
+// three tiles, the GEMM and the form taken: 1000 tokens of 8192 x 2048 54.8, 59.0 and 48.3 us
+// (two), 580 of 12288 x 2048 54.2, 56.1 and 47.3 (two), 896 of 8192 x 4096 97, 98 and 82 (two),
+// 512 of 8192 x 4096 55, 63 and 50 (one). Two rounds of them are rarely the fastest.
+static bool dense_one_round(const Matrix *m, int tokens, double pass, DensePlan &plan) {
+    if (tokens <= 256) return false;   // (not measured)
+    bool taken = false;
+    for (int slabs = 1; slabs <= 2; slabs++) {
+        const size_t row_tiles = ((size_t)m->rows + 128 * slabs - 1) / (128 * slabs);
+        if (row_tiles * (((size_t)tokens + 127) / 128) > 256) continue;
+        const double step = slabs == 2 ? (m->bits == 8 ? 1.03 : 1.13) : (m->bits == 8 ? 0.61 : 0.645);
+        const double t = 9.1 + (m->columns / 64) * step + dense_store_pass(m, tokens);
+        if (t >= (taken ? pass : pass * (slabs == 2 ? 0.95 : 0.92))) continue;
+        taken = true;
+        pass = t;
+        plan.nt = 4;
+        plan.slabs = slabs;
+        plan.ksplit = 1;
+    }
+    return taken;
 }
 
 // One dequantization pass and the bf16 GEMM of gemm.hip: a round of 256 tiles costs its shape's
@@ -955,7 +1003,7 @@ DensePlan dense_plan(const Matrix *m, int tokens, size_t part_bytes, bool ordere
     }
     const size_t row_tiles = (size_t)(m->rows + 127) / 128;
     const int windows = m->columns / 256;   // of four K steps
-    double cost = 0, pass = 0;
+    double cost = 0, pass = 0;   // pass: of a whole pass, as the forms are compared with each other
     for (int nt = 1; nt <= kDenseTiles; nt++) {
         const size_t chunks = ((size_t)tokens + 32 * nt - 1) / (32 * nt), items = row_tiles * chunks;
         const size_t plane = items * 128 * 32 * (size_t)nt * 4;
@@ -968,15 +1016,17 @@ DensePlan dense_plan(const Matrix *m, int tokens, size_t part_bytes, bool ordere
                 cost = c;
                 best.nt = nt;
                 best.ksplit = ranges;
-                if (may_gemm) pass = dense_fused_pass(m, tokens, items, nt, 4 * per, ranges, plane);
+                pass = dense_fused_pass(m, tokens, items, nt, 4 * per, ranges, plane);
             }
         }
     }
+    const double gemm = may_gemm ? dense_gemm_pass(m, tokens) : HUGE_VAL;
+    if (dense_one_round(m, tokens, std::min(pass, gemm), best)) return best;
     // The GEMM where it is the faster by estimate; 3 % are left to it for the estimates' errors.
     // Over the fit's 1,220 cases from 512 tokens on, the launch taken is 11 % faster than the GEMM on average
     // and behind it by more than 3 % in 15 (worst 9 %): 1280 tokens of a 2048 x 4096 8-bit
     // matrix 61 us as a GEMM and 44 fused, 4096 tokens of 12288 x 2048 194 and 283.
-    best.gemm = may_gemm && (best.nt == 0 || dense_gemm_pass(m, tokens) < 1.03 * pass);
+    best.gemm = gemm < 1.03 * pass;
     return best;
 }
 
@@ -984,6 +1034,8 @@ DensePlan dense_plan(const Matrix *m, int tokens, size_t part_bytes, bool ordere
 static bool launch_dense_split(const QmmArgs &a, QmmParams P, hipStream_t s, char *error, int capacity) {
     const Matrix *m = a.m0;
     const int G = m->columns >> 6, nt = a.plan.nt, chunks = (a.tokens + 32 * nt - 1) / (32 * nt);
+    const int slabs = a.plan.slabs;
+    P.row_tiles = (m->rows + 128 * slabs - 1) / (128 * slabs);
     P.ksteps = 4 * ((G / 4 + a.plan.ksplit - 1) / a.plan.ksplit);
     P.ksplit = (G + P.ksteps - 1) / P.ksteps;   // (no empty range)
     P.rtb = 1;
@@ -1006,13 +1058,14 @@ static bool launch_dense_split(const QmmArgs &a, QmmParams P, hipStream_t s, cha
     }
     const dim3 grid((unsigned)P.row_tiles, (unsigned)P.ksplit, (unsigned)chunks);
     bool found = false;
-#define DIH_DENSE_CASE(B, N)                                                                           \
-    if (m->bits == B && nt == N) {                                                                     \
-        DIH_LAUNCH((qmm_lds_kernel<B, false, N, 4, false, B == 5, N, 4>), grid, dim3(256), 0, s, P);   \
-        found = true;                                                                                  \
+#define DIH_DENSE_CASE(B, N, RS)                                                                         \
+    if (m->bits == B && nt == N && slabs == RS && (RS == 1 || P.ksplit == 1)) {                          \
+        DIH_LAUNCH((qmm_lds_kernel<B, false, N, 4, false, B == 5, N, 4, RS>), grid, dim3(256), 0, s, P); \
+        found = true;                                                                                    \
     }
-    DIH_DENSE_CASE(8, 1) DIH_DENSE_CASE(8, 2) DIH_DENSE_CASE(8, 3)
-    DIH_DENSE_CASE(5, 1) DIH_DENSE_CASE(5, 2) DIH_DENSE_CASE(5, 3)
+    DIH_DENSE_CASE(8, 1, 1) DIH_DENSE_CASE(8, 2, 1) DIH_DENSE_CASE(8, 3, 1) DIH_DENSE_CASE(8, 4, 1)
+    DIH_DENSE_CASE(5, 1, 1) DIH_DENSE_CASE(5, 2, 1) DIH_DENSE_CASE(5, 3, 1) DIH_DENSE_CASE(5, 4, 1)
+    DIH_DENSE_CASE(8, 4, 2) DIH_DENSE_CASE(5, 4, 2)
 #undef DIH_DENSE_CASE
     if (!found) {
         set_error(error, capacity, "Unsupported qmm configuration");

@@ -138,7 +138,7 @@ def load():
         "dih_moe_decode_noalloc": ([P, P, P, P, P, P, P, P, E, I], I),
         "dih_moe_prefill_norm": ([P, P, I, P, P, I, P, P, P, P, E, I], I),
         "dih_dense": ([P, P, I, P, P, I, P, E, I], I),
-        "dih_dense_plan": ([I, I, I, I, I, P, P], I),
+        "dih_dense_plan": ([I, I, I, I, I, P, P, P], I),
         "dih_grouped_qmm": ([P, P, P, I, P, I, P, P, P, I, P, E, I], I),
         "dih_attention": ([P, P, I, P, P, I, P, I, P, I, I, I, I, P, E, I], I),
         "dih_attention_partition": ([I, I, I], I),
@@ -628,13 +628,14 @@ def dense(dev, m, tokens, x, y, y_dtype=F32, stream=None) -> None:
 
 
 def dense_plan(rows, columns, bits, tokens, planes=2):
-    """(route, 32-token tiles a block, K ranges) of a dense() call (dih_dense_plan): route "gemv",
+    """(route, 32-token tiles a block, 128-row slabs a block, K ranges) of a dense() call (dih_dense_plan): route "gemv",
     "fused" or "gemm"; planes 0: under capture, 1: on a caller's stream, 2: on the context's."""
-    tiles, ranges = ctypes.c_int(), ctypes.c_int()
-    route = load().dih_dense_plan(rows, columns, bits, tokens, planes, ctypes.byref(tiles), ctypes.byref(ranges))
+    tiles, slabs, ranges = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    route = load().dih_dense_plan(rows, columns, bits, tokens, planes, ctypes.byref(tiles), ctypes.byref(slabs),
+                                  ctypes.byref(ranges))
     if route < 0:
         raise ArgumentError("Invalid dense projection arguments")
-    return ("gemv", "fused", "gemm")[route], tiles.value, ranges.value
+    return ("gemv", "fused", "gemm")[route], tiles.value, slabs.value, ranges.value
 
 
 def attention(dev, q, keys, values, gate, out, position, tokens, partition=0, q_dtype=F32,

@@ -94,7 +94,7 @@ def stable_top8(values):
 
 
 # Dense projections (rows, columns, tokens) of short and medium chunks: K in one and several ranges,
-# whole and with a shorter last one, in each width of the blocks; rows past and off the
+# whole and with a shorter last one, in each width of the blocks, and two slabs a wave; rows past and off the
 # 128-row tiles and not whole float4, tokens past and off the 32-token tiles; the last two of the
 # first block are past the GEMM's first token count.
 DENSE_FUSED_SHAPES = [
@@ -102,7 +102,7 @@ DENSE_FUSED_SHAPES = [
     (1003, 2048, 97), (2048, 512, 128), (513, 1536, 129), (4100, 512, 160), (512, 8192, 193), (300, 2560, 300),
     (8192, 512, 700), (512, 2048, 1300), (2048, 1024, 1500),
     (8192, 2560, 5), (4099, 5120, 33), (2045, 5120, 129), (2500, 512, 400), (4100, 1024, 33), (2500, 4608, 65),
-    (129, 6656, 300)]
+    (129, 6656, 300), (8188, 2048, 970), (8188, 4096, 490)]
 
 # (bits, rows, columns, tokens, bf16 rows, the GEMM's block: rows x tokens): each block shape with
 # ragged row and token tiles, rows in and off 16-byte pieces.

@@ -725,7 +725,7 @@ def _dense_route(device, run):
 @pytest.mark.parametrize("bits,rows,columns,T,y_bf16,route", [
     (8, 300, 512, 1024, False, "fused"), (8, 2048, 4096, 512, True, "split"), (5, 1000, 2048, 1100, False, "split"),
     (5, 64, 256, 2048, True, "gemm"), (8, 4100, 1024, 512, False, "fused"),   # (past 4096 rows: from 1024 tokens)
-    (8, 300, 448, 1024, False, "gemm"), (8, 2048, 4032, 512, True, "gemm"), (8, 4096, 4096, 2048, True, "gemm")])
+    (8, 300, 448, 1024, False, "gemm"), (8, 2048, 4032, 512, True, "gemm"), (8, 4096, 4096, 2100, True, "gemm")])
 def test_dense_long_chunks(device, bits, rows, columns, T, y_bf16, route):
     """Long chunks (1024 tokens and more, or 512 and more for matrices of up to 4096 rows)
     run fused or as one dequantization pass into bf16 and a bf16 GEMM with f32 accumulation
@@ -781,10 +781,13 @@ def test_dense_gemm_tile_shapes(device, bits, rows, columns, T, y_bf16, block):
         m.dispose()
 
 
-@pytest.mark.parametrize("bits,rows,columns,T", [(8, 16384, 512, 512), (5, 16400, 512, 520)])
-def test_dense_many_row_tiles(device, bits, rows, columns, T):
-    """Chunks of matrices with 128 row tiles and more (several rounds of blocks); ragged rows and
-    tokens included."""
+@pytest.mark.parametrize("bits,rows,columns,T,slabs", [
+    (8, 16384, 512, 512, 2), (5, 16400, 512, 520, 1), (8, 8192, 2048, 1000, 2), (5, 8100, 2048, 900, 2),
+    (8, 8004, 2048, 960, 2), (5, 16300, 2048, 450, 2), (8, 12200, 2048, 545, 2)])
+def test_dense_two_slab_tiles(device, bits, rows, columns, T, slabs):
+    """Dense launches in one round of 256-row tiles, two 32-row slabs a wave; ragged rows and
+    tokens (one to four 32-token tiles in the last chunk) included; one shape of many one-slab tiles."""
+    assert dh.dense_plan(rows, columns, bits, T)[:3:2] == ("fused", slabs)
     rng = np.random.default_rng(rows + T)
     host = orc.random_matrix(rng, 1, rows, columns, bits)
     m = upload(device, host)
@@ -793,7 +796,7 @@ def test_dense_many_row_tiles(device, bits, rows, columns, T):
         y = torch.zeros((T, rows), dtype=torch.float32, device="cuda")
         dh.dense(device, m, T, dev_bf16(xb), y)
         torch.cuda.synchronize()
-        want_bf = orc.dense_f64(host, orc.bf16_bits_to_f32(xb), round_operands=True)
+        want_bf = orc.dense_f64_blas(host, orc.bf16_bits_to_f32(xb), round_operands=True)
         assert orc.rel_err(y.cpu().numpy(), want_bf) < 1e-4
     finally:
         m.dispose()
@@ -812,7 +815,7 @@ def test_dense_split_ranges(device, bits, rows, columns, T):
         xb = orc.f32_to_bf16_bits(rng.normal(size=(T, columns)).astype(np.float32))
         y = torch.full((T + 1, rows), 7.0, dtype=torch.float32, device="cuda")
         yb = torch.full((T + 1, rows), 7, dtype=torch.int16, device="cuda")
-        ranges = dh.dense_plan(rows, columns, bits, T)[2]
+        ranges = dh.dense_plan(rows, columns, bits, T)[3]
         route = _dense_route(device, lambda: dh.dense(device, m, T, dev_bf16(xb), y))
         assert route == ("split" if ranges > 1 else "fused")
         dh.dense(device, m, T, dev_bf16(xb), yb, y_dtype=dh.BF16)
@@ -865,7 +868,7 @@ def test_dense_short_chunks_on_streams_and_in_graphs():
         m.dispose()
 
 
-@pytest.mark.parametrize("rows,columns,T", [(8192, 4096, 1024), (512, 2048, 4096)])
+@pytest.mark.parametrize("rows,columns,T", [(8192, 4096, 1100), (512, 2048, 4096)])
 def test_dense_long_chunk_captured_first(rows, columns, T):
     """A chunk that runs as the GEMM can be captured as its context's first call, where the weight
     copy cannot be allocated (it then stays on the fused kernel), and after an eager call."""
