@@ -327,7 +327,7 @@ __global__ __launch_bounds__(256, 3) void delta_prepare_kernel(DeltaParams P) {
                 ti[(o == 0 ? t : t + 16) * kSq4 + (o == 0 ? 16 + c : c)] = 0.f;   // T12 = 0; T21 below
             }
         }
-        wait_lgkm0();
+        wave_fence();
         // step s covers k = 4g + s (lane group g = lane / 16), so the product M = L21 T11 in
         // its accumulator layout (register s: row 4g + s) is the B operand of the next
         const int n = lane & 15, g = lane >> 4;
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(256, 3) void delta_prepare_kernel(DeltaParams P) {
         // of W~ and Q', tokens 16tt + 4g ..+3 of dim 32w + 16mt + n of K, at
         // [w][tt][mt][lane][4]: every load there is 1 KB on end. K once a key head, by its
         // even value head. W~ and Q' change order through this wave's own columns of ks and qs,
-        // which no other wave reads any more, so there is no barrier.
+        // which no other wave reads any more: the wave's own order is enough.
         const int n = lane & 15, g = lane >> 4, at = wave * 1024 + 4 * lane;
         if (!(head & 1)) {
             float *kt = P.kf + ((size_t)blk * (kVHeads / 2) + kh) * (kBlk * kDim) + at;
@@ -395,6 +395,7 @@ __global__ __launch_bounds__(256, 3) void delta_prepare_kernel(DeltaParams P) {
             ks[t * kPad4 + dcol] = tl[t] * wa[i];
             qs[t * kPad4 + dcol] = gs[t] * qs[t * kPad4 + dcol] - cw[i];
         }
+        wave_fence();
         float *wt = P.w + tile * (kBlk * kDim) + at, *qt = P.qp + tile * (kBlk * kDim) + at;
 #pragma unroll
         for (int f = 0; f < 4; f++) {

@@ -310,6 +310,13 @@ DIH_DEV void wait_lgkm0() { __builtin_amdgcn_s_waitcnt((15) | (7 << 4) | (0 << 8
 // for LDS arrays that have escaped (see lds_escape).
 DIH_DEV void barrier_no_fence() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// Between LDS stores and reads by other lanes of the same wave. The hardware keeps a wave's LDS
+// operations in order; this keeps the compiler to that order (no instruction).
+DIH_DEV void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Makes LDS arrays escape, so that alias analysis treats them as memory that an asm with a
 // "memory" clobber (barrier_no_fence) may touch; without it a __shared__ array that never
 // escapes can have its accesses reordered across such an asm.
