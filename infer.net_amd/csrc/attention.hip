@@ -494,9 +494,8 @@ __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
     uint32_t pw[8];
     // Copy i of a tile's keys (or values) by this wave: rows 4 * wave + 2i and the next one, from
     // the block's first key on, a lane 16 bytes; rows past the partition's end repeat its last
-    // key (finite data; those keys are masked). Untracked by the compiler (as copy16_to_lds,
-    // without a memory clobber: nothing reads the slot before the barrier the copies are waited
-    // for at): it would make the first operand read of a step wait for the copies just issued.
+    // key (finite data; those keys are masked). Untracked by the compiler (copy16_to_lds), which
+    // would make the first operand read of a step wait for the copies just issued.
     const uint16_t *const kfirst = kbase + (size_t)kstart * (kKvHeads * kDim);
     const uint16_t *const vfirst = vbase + (size_t)kstart * (kKvHeads * kDim);
     const uint32_t ks_lds = (uint32_t)(uintptr_t)&ks[0][0], vs_lds = (uint32_t)(uintptr_t)&vs[0][0];
@@ -505,9 +504,7 @@ __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
         const int kl = 4 * wave + 2 * i + (l >> 5);
         const uint32_t c = (uint32_t)((l & 31) ^ (keys ? kl & 15 : 4 * (kl & 3)));
         const uint32_t row = (uint32_t)min(j * kKeys + kl, kend - kstart - 1);
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(row << 10 | c << 4),
-                     "s"(base), "s"(slot + (uint32_t)(4 * wave + 2 * i) * (kDim * 2))
-                     : "m0");
+        copy16_to_lds<false>(base, row << 10 | c << 4, slot + (uint32_t)(4 * wave + 2 * i) * (kDim * 2));
     };
     static_assert(kKvHeads * kDim * 2 == 1 << 10, "bytes of a cache row");
     auto keys = [&](int j, int slot) {

@@ -285,10 +285,17 @@ DIH_DEV void to_lds(const void *src, void *lds_wave_base) {
 // so that the compiler does not track these LDS writes: it would otherwise make every LDS
 // read wait for all copies in flight, since it cannot tell the stages apart. The kernels
 // order the copies themselves (vmcnt waits on their own copies, then a barrier, before a
-// stage is read).
+// stage is read). FENCE false: without a memory clobber, for copies issued between the reads of
+// other slots, where nothing reads the copy's own slot before the barrier that it is waited
+// for at.
+template <bool FENCE = true>
 DIH_DEV void copy16_to_lds(const void *base, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
-                 : "memory", "m0");
+    if constexpr (FENCE)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+                     : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds)
+                     : "m0");
 }
 
 // s_waitcnt vmcnt(N) leaving the other counters alone (gfx9 encoding)

@@ -443,20 +443,13 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
         first = (int)blockIdx.z * BN;
         nvalid = min(BN, P.tokens - first);
     } else {
-        const int chunks = P.dense ? (P.tokens + BN - 1) / BN : chunk_total<BN>(P.counts, P.ngroups);
+        const int chunks = chunk_total<BN>(P.counts, P.ngroups);
         const int L = xcd_item((int)blockIdx.x, chunks * P.rt_groups);
         const int ci = L < 0 ? chunks : L / P.rt_groups;
-        bool ok;
-        if (P.dense) {
-            ok = L >= 0 && ci * BN < P.tokens;
-            if (ok) { first = ci * BN; nvalid = min(BN, P.tokens - first); }
-        } else {
-            int count;
-            const int total = chunk_of<BN>(P.counts, P.ngroups, ci, e, first, count);
-            ok = L >= 0 && ci < total;
-            if (ok) nvalid = min(BN, count - first);
-        }
-        if (ok) {
+        int count;
+        const int total = chunk_of<BN>(P.counts, P.ngroups, ci, e, first, count);
+        if (L >= 0 && ci < total) {
+            nvalid = min(BN, count - first);
             rt0 = (L - ci * P.rt_groups) * P.rtb;
             nrt = min(P.rtb, P.row_tiles - rt0);
         }
@@ -477,11 +470,11 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
     // route of the chunk's n-th slot (slots past the chunk repeat its first route)
     auto route_at = [&](int n) -> int {
         n = n < nvalid ? n : 0;
-        return KS == 4 || P.dense ? first + n : (int)P.routes[(size_t)e * P.tokens + first + n];
+        return KS == 4 ? first + n : (int)P.routes[(size_t)e * P.tokens + first + n];
     };
 
     // ---- weights
-    const bool shared = KS != 4 && !P.dense && e == P.experts;
+    const bool shared = KS != 4 && e == P.experts;
     const char *pw[2] = {reinterpret_cast<const char *>(shared ? P.sp0 : P.p0),
                          reinterpret_cast<const char *>(shared ? P.sp1 : P.p1)};
     const uint16_t *psc[2] = {shared ? P.ss0 : P.s0, shared ? P.ss1 : P.s1};
@@ -1092,7 +1085,7 @@ bool launch_qmm(const QmmArgs &a, hipStream_t s, char *error, int capacity) {
     P.ngroups = a.ngroups;
     P.routes = a.routes; P.counts = a.counts;
     P.x = a.x; P.y = a.y;
-    if (!a.dense && (a.ngroups < 1 || a.ngroups > 320 || !a.routes || !a.counts)) {
+    if (a.dense ? m1 != nullptr : a.ngroups < 1 || a.ngroups > 320 || !a.routes || !a.counts) {
         set_error(error, capacity, "Invalid grouped qmm arguments");
         return false;
     }
@@ -1116,14 +1109,13 @@ bool launch_qmm(const QmmArgs &a, hipStream_t s, char *error, int capacity) {
     // - other K (the register-ring kernel): 64 gated, 128 otherwise.
     const bool gated = m1 != nullptr;
     const bool streaming = m0->columns % 512 == 0;
-    if (streaming && a.dense && !gated) return launch_dense_split(a, P, s, error, capacity);
-    const bool grouped = streaming && !a.dense;
+    if (streaming && a.dense) return launch_dense_split(a, P, s, error, capacity);
     const size_t routes = (size_t)a.tokens * 8, experts = (size_t)std::max(1, m0->experts);
     const bool five = m0->bits == 5;
     int nt = gated ? 2 : 4;
-    if (grouped && gated) nt = qmm_wide_gated(m0, a.tokens) ? 4 : routes <= (five ? 24 : 8) * experts ? 1 : 2;
-    if (grouped && !gated) nt = five && routes > 48 * experts ? 3 : routes <= (five ? 24 : 16) * experts ? 1 : 2;
-    const int ntc = nt == 4 && grouped && gated && routes <= 64 * experts ? 3 : nt;
+    if (streaming && gated) nt = qmm_wide_gated(m0, a.tokens) ? 4 : routes <= (five ? 24 : 8) * experts ? 1 : 2;
+    if (streaming && !gated) nt = five && routes > 48 * experts ? 3 : routes <= (five ? 24 : 16) * experts ? 1 : 2;
+    const int ntc = nt == 4 && streaming && gated && routes <= 64 * experts ? 3 : nt;
     const int bn = 32 * ntc;
     const size_t work = qmm_max_work(m0->rows, a.tokens, a.ngroups, a.dense, bn);
     const size_t blocks = 8 * ((work + 7) / 8);
