@@ -895,12 +895,13 @@ static int dense_resident(int bits, int nt) {
     return kResident[bits == 8][nt];
 }
 
-// The estimate dense_plan minimizes, in us, fitted to 770 measured launches (four model
+// The estimate dense_plan minimizes, in us, fitted to 770 measured kernels (four model
 // projections, 5 and 8 bits, 16 to 1023 tokens; median error 5 %, and the plan it picks is
 // 0.5 % behind the best one on average, 7 % at worst). n blocks of nt 32-token tiles run on
 // each CU, `resident` at a time; a K step of c resident blocks takes the larger of one
-// block's latency and c times its issue time. Ranges add the sum pass: its launch, the
-// planes' write and read and, with planes ordered by events (`ordered`), the event's record
+// block's latency and c times its issue time. Ranges add the sum pass: its launch (unsplit and
+// split, among other passes: 16 tokens of 2048 x 512 5.6 and 8.5 us, of 2048 x 1024 8.3 and
+// 9.0, of 512 x 1536 11.0 and 9.3, of 512 x 2048 13.7 and 9.2), the planes' write and read and, with planes ordered by events (`ordered`), the event's record
 // and its gap (split on the context's stream, split on another, unsplit: 61 tokens of a
 // 2048 x 4096 matrix 11.5, 16.9 and 23.6 us, 16 tokens of 8192 x 2048 10.2, 14.9 and 13.0,
 // 64 tokens of 512 x 2048 9.4, 15.7 and 13.1: the last two run unsplit there).
@@ -911,7 +912,7 @@ static double dense_cost(int bits, size_t items, int nt, int steps, int ksplit, 
     const auto round = [&](size_t c) { return 0.755 + slow * steps * std::max(latency, issue * (double)c); };
     double t = 4.3 + (double)(n / resident) * round(resident);
     if (n % resident) t += round(n % resident);
-    return ksplit > 1 ? t + (ordered ? 9.0 : 0.78) + (double)ksplit * (double)plane_bytes * 2.0 / 5.0e6 : t;
+    return ksplit > 1 ? t + (ordered ? 9.0 : 1.5) + (double)ksplit * (double)plane_bytes * 2.0 / 5.0e6 : t;
 }
 
 // From 512 tokens on the choice between the fused launch and the GEMM has estimates of its own,

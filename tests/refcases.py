@@ -102,7 +102,7 @@ DENSE_FUSED_SHAPES = [
     (1003, 2048, 97), (2048, 512, 128), (513, 1536, 129), (4100, 512, 160), (512, 8192, 193), (300, 2560, 300),
     (8192, 512, 700), (512, 2048, 1300), (2048, 1024, 1500),
     (8192, 2560, 5), (4099, 5120, 33), (2045, 5120, 129), (2500, 512, 400), (4100, 1024, 33), (2500, 4608, 65),
-    (129, 6656, 300), (8188, 2048, 970), (8188, 4096, 490)]
+    (129, 6656, 300), (2045, 5632, 65), (8188, 2048, 970), (8188, 4096, 490)]
 
 # (bits, rows, columns, tokens, bf16 rows, the GEMM's block: rows x tokens): each block shape with
 # ragged row and token tiles, rows in and off 16-byte pieces.

@@ -50,6 +50,17 @@ def test_refused_arguments():
             dh.dense_plan(*args)
 
 
+# Measured microseconds of a pass (one range, the best ranges): the second launch costs more than
+# ranges give where K is short.
+@pytest.mark.parametrize("bits,rows,columns,tokens,one,split", [
+    (8, 512, 512, 16, 5.8, 9.0), (8, 2048, 512, 64, 5.6, 8.7), (8, 4100, 512, 33, 5.7, 8.7),
+    (8, 8192, 512, 128, 6.5, 12.5), (8, 8192, 1024, 33, 8.7, 9.9), (8, 2048, 1024, 256, 8.9, 10.7),
+    (8, 512, 1536, 16, 11.0, 9.3), (8, 512, 2048, 64, 14.0, 9.1), (8, 2048, 2048, 128, 14.2, 11.2),
+    (8, 8192, 2048, 16, 14.0, 9.9)])
+def test_ranges_where_they_pay(bits, rows, columns, tokens, one, split):
+    assert (dh.dense_plan(rows, columns, bits, tokens)[3] > 1) == (split < one)
+
+
 # Measured microseconds of a pass: blocks of 128 tokens and one or two 32-row slabs a wave fill the
 # GPU in one round where the narrower blocks cross it.
 @pytest.mark.parametrize("bits,rows,columns,tokens,slabs,narrow,wide", [

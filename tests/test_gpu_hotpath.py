@@ -725,7 +725,7 @@ def _dense_route(device, run):
 @pytest.mark.parametrize("bits,rows,columns,T,y_bf16,route", [
     (8, 300, 512, 1024, False, "fused"), (8, 2048, 4096, 512, True, "split"), (5, 1000, 2048, 1100, False, "split"),
     (5, 64, 256, 2048, True, "gemm"), (8, 4100, 1024, 512, False, "fused"),   # (past 4096 rows: from 1024 tokens)
-    (8, 300, 448, 1024, False, "gemm"), (8, 2048, 4032, 512, True, "gemm"), (8, 4096, 4096, 2100, True, "gemm")])
+    (8, 300, 448, 1024, False, "gemm"), (8, 2048, 4032, 512, True, "gemm"), (8, 6000, 2048, 2100, True, "gemm")])
 def test_dense_long_chunks(device, bits, rows, columns, T, y_bf16, route):
     """Long chunks (1024 tokens and more, or 512 and more for matrices of up to 4096 rows)
     run fused or as one dequantization pass into bf16 and a bf16 GEMM with f32 accumulation
@@ -868,7 +868,7 @@ def test_dense_short_chunks_on_streams_and_in_graphs():
         m.dispose()
 
 
-@pytest.mark.parametrize("rows,columns,T", [(8192, 4096, 1100), (512, 2048, 4096)])
+@pytest.mark.parametrize("rows,columns,T", [(6001, 2048, 2100), (512, 2048, 4096)])
 def test_dense_long_chunk_captured_first(rows, columns, T):
     """A chunk that runs as the GEMM can be captured as its context's first call, where the weight
     copy cannot be allocated (it then stays on the fused kernel), and after an eager call."""
