@@ -439,13 +439,14 @@ DIH_DEV void multiply_tile(uint32_t vs, uint32_t ks, const uint32_t (&pw)[8], co
 // ---- eight-wave form: 32 query tokens (256 rows) per block share each key/value tile. Waves
 // w and w + 4 share a SIMD, and the two groups run the same loop half a step apart: while one
 // group's wave multiplies (V^T P^T of tile j, then K Q^T of tile j + 1), the other's computes a
-// softmax, with a barrier at every change. Bound by the two halves, 1,500-1,800 cycles each of
-// a tile's 4,150: the softmax by its VALU work (121 instructions, 16 exponentials among them,
-// and 128 multiplies where a row's scale moves), the products by MFMAs (1,024) and the latency
-// of their operand reads. In lockstep, with one accumulator set and its spills, MFMAs, LDS
-// reads, softmax and the values' transposition took turns: 7,500 cycles a tile. The last
-// 2048-token chunk of a 32K prompt 1,610 -> 1,099 us, 2048 tokens from position 0 119 -> 98
-// us, 837 tokens at position 18,686 671 -> 436 us. Spreading the rescale over the MFMAs, two
+// softmax, with a barrier at every change. Bound by the two halves together, 3,870 cycles a tile:
+// the softmax by its VALU work (121 instructions, 16 exponentials among them, and 128
+// multiplies where a row's scale moves), the products by MFMAs (1,024 cycles a wave: the pipe
+// is busy 51 % of the time) and the latency of their operand reads. In lockstep, with one
+// accumulator set and its spills, MFMAs, LDS reads, softmax and the values' transposition took
+// turns: 7,450 cycles a tile, pipe busy 27 %. The last 2048-token chunk of a 32K prompt 1,610
+// -> 1,000-1,110 us (by the box), 2048 tokens from position 0 119 -> 98 us, 837 tokens at
+// position 18,686 671 -> 436 us. Spreading the rescale over the MFMAs, two
 // score chains and alternating the products were each no faster (more registers, so shorter
 // operand read-ahead).
 // Keys and values are triple-buffered raw rows: step j reads values j and keys j + 1, and

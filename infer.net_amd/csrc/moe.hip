@@ -160,8 +160,8 @@ bool launch_build_groups(const uint32_t *ids, int tokens, int experts, int with_
 // barrier they then cover, and a row of up to kMergeHold pieces keeps its stored r in
 // registers for the norm. VEC 4 needs every row 16-byte aligned (8-byte for bf16), VEC 1
 // takes any other caller buffers. Against one column a thread at a time behind the gate: a
-// 77-token 5-bit layer with norm 143.2 -> 138.6 us, 2048 tokens 349.9 -> 343.6 us, 512 tokens
-// without norm 243.5 -> 241.5 us.
+// 77-token 5-bit layer with norm 143.2 -> 138.6 us, 2048 tokens 349.9 -> 343.6 us; a 512-token
+// 8-bit one within the runs' spread.
 constexpr int kMergeHold = 2;
 
 // VEC consecutive elements of an f32 or bf16 row.

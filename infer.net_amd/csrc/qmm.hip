@@ -543,10 +543,10 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256, (qmm_lds_waves<BITS, GATED, NT, 
     // offset of the row within the expert (an expert's rows span less than 2^31 bytes, checked
     // on the host); a K step adds the wave-uniform offset kg * KSTEP. Row-major codes: a row
     // starts row * row_bytes in, a K step is AB bytes further. Tile-major codes (experts padded
-    // to whole 256-row tiles, so a 256-row dense tile stays inside the copy): a 128-row tile starts tile * 128 * row_bytes in, its row rr
-    // rr * AB further, and a K step is 128 * AB bytes. The issue position (the next step to
-    // copy, as tile and K step) is wave-uniform, so the step bookkeeping is scalar and no step
-    // index is divided at run time.
+    // to whole 256-row tiles, so a 256-row dense tile stays inside the copy): a 128-row tile
+    // starts tile * 128 * row_bytes in, its row rr rr * AB further, and a K step is 128 * AB
+    // bytes. The issue position (the next step to copy, as tile and K step) is wave-uniform, so
+    // the step bookkeeping is scalar and no step index is divided at run time.
     constexpr uint32_t KSTEP = TL ? 128 * AB : AB;
     const size_t wrows = TL ? (size_t)((R + 255) & ~255) : (size_t)R;  // code rows per expert
     const char *wbase[WMAT];
@@ -895,16 +895,17 @@ static int dense_resident(int bits, int nt) {
     return kResident[bits == 8][nt];
 }
 
-// The estimate dense_plan minimizes, in us, fitted to 770 measured kernels (four model
-// projections, 5 and 8 bits, 16 to 1023 tokens; median error 5 %, and the plan it picks is
-// 0.5 % behind the best one on average, 7 % at worst). n blocks of nt 32-token tiles run on
-// each CU, `resident` at a time; a K step of c resident blocks takes the larger of one
-// block's latency and c times its issue time. Ranges add the sum pass: its launch (unsplit and
-// split, among other passes: 16 tokens of 2048 x 512 5.6 and 8.5 us, of 2048 x 1024 8.3 and
-// 9.0, of 512 x 1536 11.0 and 9.3, of 512 x 2048 13.7 and 9.2), the planes' write and read and, with planes ordered by events (`ordered`), the event's record
-// and its gap (split on the context's stream, split on another, unsplit: 61 tokens of a
-// 2048 x 4096 matrix 11.5, 16.9 and 23.6 us, 16 tokens of 8192 x 2048 10.2, 14.9 and 13.0,
-// 64 tokens of 512 x 2048 9.4, 15.7 and 13.1: the last two run unsplit there).
+// The estimate that ranks the fused forms, in us, fitted to 770 measured kernels (four model
+// projections, 5 and 8 bits, 16 to 1023 tokens; median error 5 %). Over 1,596 passes of 19
+// shapes and up to 500 tokens the form it picks is 2.7 % behind the best one on average. n
+// blocks of nt 32-token tiles run on each CU, `resident` at a time; a K step of c resident
+// blocks takes the larger of one block's latency and c times its issue time. Ranges add the
+// planes' write and read and the sum pass's launch (unsplit and split, among other passes: 16
+// tokens of 2048 x 512 5.6 and 8.5 us, of 2048 x 1024 8.3 and 9.0, of 512 x 1536 11.0 and 9.3,
+// of 512 x 2048 13.7 and 9.2) or, with planes ordered by events (`ordered`), that and the event's
+// record and gap (split on the context's stream, split on another, unsplit: 61 tokens of
+// 2048 x 4096 11.5, 16.9 and 23.6 us, 16 of 8192 x 2048 10.2, 14.9 and 13.0, 64 of 512 x 2048
+// 9.4, 15.7 and 13.1: the last two run unsplit there).
 static double dense_cost(int bits, size_t items, int nt, int steps, int ksplit, size_t plane_bytes, bool ordered) {
     const int resident = dense_resident(bits, nt);
     const double slow = bits == 8 ? 1.0 : 1.1, latency = 0.2 + 0.111 * nt, issue = 0.185 + 0.054 * nt;
@@ -1017,14 +1018,15 @@ DensePlan dense_plan(const Matrix *m, int tokens, size_t part_bytes, bool ordere
     const double gemm = may_gemm ? dense_gemm_pass(m, tokens) : HUGE_VAL;
     if (dense_one_round(m, tokens, std::min(pass, gemm), best)) return best;
     // The GEMM where it is the faster by estimate; 3 % are left to it for the estimates' errors.
-    // Over the fit's 1,220 cases from 512 tokens on, the launch taken is 11 % faster than the GEMM on average
-    // and behind it by more than 3 % in 15 (worst 9 %): 1280 tokens of a 2048 x 4096 8-bit
-    // matrix 61 us as a GEMM and 44 fused, 4096 tokens of 12288 x 2048 194 and 283.
+    // Over the fit's 1,220 cases from 512 tokens on, the launch taken is 11 % faster than the
+    // GEMM on average and behind it by more than 3 % in 15 (worst 9 %): 1280 tokens of a 2048 x
+    // 4096 8-bit matrix 61 us as a GEMM and 44 fused, 4096 tokens of 12288 x 2048 194 and 283.
     best.gemm = gemm < 1.03 * pass;
     return best;
 }
 
-// A dense streaming launch as planned: nt 32-token tiles a block, K in ksplit ranges.
+// A dense streaming launch as planned: nt 32-token tiles and 128 * slabs rows a block, K in
+// ksplit ranges.
 static bool launch_dense_split(const QmmArgs &a, QmmParams P, hipStream_t s, char *error, int capacity) {
     const Matrix *m = a.m0;
     const int G = m->columns >> 6, nt = a.plan.nt, chunks = (a.tokens + 32 * nt - 1) / (32 * nt);
