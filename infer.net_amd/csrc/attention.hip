@@ -456,7 +456,7 @@ DIH_DEV void multiply_tile(uint32_t vs, uint32_t ks, const uint32_t (&pw)[8], co
 template <bool RESTARTS>
 __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
     __shared__ __align__(16) uint16_t ks[3][kKeys * kDim];
-    __shared__ __align__(16) uint16_t vs[4][kKeys * kDim];   // (the fourth: zeros)
+    __shared__ __align__(16) uint16_t vs[3][kKeys * kDim];
     lds_escape(ks, vs);
 
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, r = lane & 31, h = lane >> 5;
@@ -472,9 +472,6 @@ __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
     if (kstart >= kend) return;
 
     const int wtok0 = tok0 + 4 * wave;
-#pragma unroll
-    for (int i = 0; i < kKeys * kDim / (8 * 512); i++)
-        *reinterpret_cast<uint4 *>(&vs[3][8 * (t + 512 * i)]) = make_uint4(0, 0, 0, 0);
     dih_bf16x8 qreg[16];
     load_queries(qreg, P, wtok0 + (r >> 3), wtok0 + (r >> 3) < P.tokens, kh * kGroup + (r & 7), h);
     RowState st;
@@ -486,11 +483,13 @@ __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
 
     const uint16_t *kbase = P.keys + kh * kDim, *vbase = P.values + kh * kDim;
     const int ntile = (kend - kstart + kKeys - 1) / kKeys;
-    // Tiles up to the wave's last visible key. Those behind have probabilities of 0 for all of the
-    // wave's rows, but 0 times a NaN or an infinity of a later token's value row would still be
-    // NaN: the wave multiplies them as zeros (a slot's number, where a branch around the
-    // products costs 288 spilled registers).
-    const int visible = (P.position + min(wtok0 + 3, P.tokens - 1) - kstart + kKeys) / kKeys;
+    // Tiles up to the wave's last visible key (none for a wave past the chunk). Those behind have
+    // probabilities of 0 for all of the wave's rows, but 0 times a NaN or an infinity of a later
+    // token's value row would still be NaN: the wave only copies and waits for them, in a loop of
+    // its own (a branch around the products costs 288 spilled registers, a slot of zeros to
+    // multiply instead 0.8-1 us a call).
+    const int visible =
+        wtok0 < P.tokens ? min(ntile, (P.position + min(wtok0 + 3, P.tokens - 1) - kstart + kKeys) / kKeys) : 0;
     dih_f32x16 s;
     uint32_t pw[8];
     // Copy i of a tile's keys (or values) by this wave: rows 4 * wave + 2i and the next one, from
@@ -522,8 +521,8 @@ __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
         asm volatile("" : "+v"(l));
         return l;
     };
-    // (every wave takes part in every tile: rows that see none of its keys have masked scores,
-    // which leave their state as it is; for the products see `visible`)
+    // (rows that see none of a tile's keys have masked scores, which leave their state and
+    // accumulators as they are)
     auto soften = [&](int j) {
         const int kb = kstart + j * kKeys;
         const bool full = kb + kKeys - 1 <= P.position + wtok0 && kb + kKeys <= kend;
@@ -548,24 +547,32 @@ __global__ __launch_bounds__(512, 1) void attn8_kernel(AttnParams P) {
     flip();
     int s0 = 0, s1 = 1, s2 = 2;   // slots of tiles j, j + 1, j + 2
     if (wave >= 4) flip();        // the second group runs one phase behind
-    for (int j = 0; j < ntile; j++) {
-        // (formed ahead of the softmax: scalar work between a flip and the first operand read
-        // is time on the chain)
-        uint32_t vtile = vs_lds + (uint32_t)(j < visible ? s0 : 3) * kSlot;
-        asm volatile("" : "+s"(vtile));
-        soften(j);
-        flip();
-        const int l = fresh();
-        multiply_tile(vtile, ks_lds + (uint32_t)s1 * kSlot, pw, qreg, acc, s, l, [&](int i) {
-            if (i < 2) copy(vfirst, vs_lds + (uint32_t)s2 * kSlot, false, j + 2, i, l);
-            else copy(kfirst, ks_lds + (uint32_t)s0 * kSlot, true, j + 3, i - 2, l);
-        });
+    const auto request = [&](int j, int i, int l) {   // copy i of the step's four
+        if (i < 2) copy(vfirst, vs_lds + (uint32_t)s2 * kSlot, false, j + 2, i, l);
+        else copy(kfirst, ks_lds + (uint32_t)s0 * kSlot, true, j + 3, i - 2, l);
+    };
+    const auto next = [&]() {
         wait_vm<4>();   // the next step's keys and values
         flip();
         const int o = s0;
         s0 = s1;
         s1 = s2;
         s2 = o;
+    };
+    int j = 0;
+    for (; j < visible; j++) {
+        soften(j);
+        flip();
+        const int l = fresh();
+        multiply_tile(vs_lds + (uint32_t)s0 * kSlot, ks_lds + (uint32_t)s1 * kSlot, pw, qreg, acc, s, l,
+                      [&](int i) { request(j, i, l); });
+        next();
+    }
+    for (; j < ntile; j++) {
+        flip();
+        const int l = fresh();
+        for (int i = 0; i < 4; i++) request(j, i, l);
+        next();
     }
     if (wave < 4) flip();
     wait_vm<0>();   // no copy may still be writing this block's LDS when the block exits
