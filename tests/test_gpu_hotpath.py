@@ -899,6 +899,36 @@ def test_dense_long_chunk_captured_first(rows, columns, T):
         m.dispose()
 
 
+def test_dense_first_split_call_beside_a_capture():
+    """A context's first split call, which allocates its planes, may run on one stream while
+    another is under capture: it neither fails nor ends the capture."""
+    rng = np.random.default_rng(63)
+    T, rows, columns = 61, 2048, 4096
+    host = orc.random_matrix(rng, 1, rows, columns, 8)
+    xb = orc.f32_to_bf16_bits(rng.normal(size=(T, columns)).astype(np.float32))
+    want = orc.dense_f64_blas(host, orc.bf16_bits_to_f32(xb), round_operands=True)
+    with dh.QuantizedHip() as dev:
+        m = upload(dev, host)
+        x, y, yg = dev_bf16(xb), torch.zeros((T, rows), device="cuda"), torch.zeros((T, rows), device="cuda")
+        other, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g):
+            dh.dense(dev, m, T, x, yg)
+            dh.dense(dev, m, T, x, y, stream=other)
+        torch.cuda.synchronize()
+        assert orc.rel_err(y.cpu().numpy(), want) < 1e-4
+        for _ in range(3):
+            yg.zero_()
+            torch.cuda.synchronize()
+            g.replay()
+            dh.dense(dev, m, T, x, y, stream=other)
+            torch.cuda.synchronize()
+            assert orc.rel_err(yg.cpu().numpy(), want) < 1e-4
+            assert orc.rel_err(y.cpu().numpy(), want) < 1e-4
+        del g
+        m.dispose()
+
+
 def test_dense_planes_on_per_thread_and_many_streams():
     """A stream handle does not identify a stream: hipStreamPerThread (handle 2) is another one
     in every thread. Threads that serialize their calls on one context and pass it, and callers
